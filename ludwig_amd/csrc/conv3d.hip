@@ -17,10 +17,9 @@
 // Backward data, dx = sum_t W_{26-t}^T dy(p + o_t): the same kernel with the
 //   weights flipped and transposed (conv3_weights_prep).
 // Backward weight, dW_t = sum_p dy(p) x(p + o_t)^T:  GEMM with M = Cout,
-//   N = Cin, K = positions; 64-position slices of dy and of the shifted x
-//   are staged through LDS (contiguous rows) and read as fragments;
-//   position chunks give partial sums that a second kernel adds in a fixed
-//   order (deterministic).
+//   N = Cin, K = positions; tiles of dy and x are staged through LDS, read as
+//   transposed fragments, and the blocks' sums are added in a fixed order
+//   (deterministic).
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -482,91 +481,237 @@ conv3_fwd_pipe_kernel(const uint16_t * __restrict__ x, const uint16_t * __restri
   }
 }
 
-constexpr int WG_P = 64;          // positions per LDS slice
-constexpr int WG_CMAX = 160;      // channel capacity of the LDS rows (host checks)
+// ---------------------------------------------------------------------------
+// Weight gradient, dW_t[co][ci] = sum_p dy(p)[co] x(p + o_t)[ci].
+//
+// One of the two arrays is read in place ("fixed", the one with more
+// channels), the other at the 27 shifted positions; shifting dy instead of x
+// only turns tap t into tap 26 - t.  A block owns 16 channels of the shifted
+// array and 16*NF of the fixed one, and marches along x over a WT_Y x WT_Z
+// (y, z) tile: LDS holds four planes of the shifted tile with its halo and
+// two of the fixed tile, so each plane is fetched once for the 27 taps and
+// the next plane's loads are in flight while the current one is used.  Wave w
+// accumulates taps 7w .. 7w+6 over all positions of the tile.
+//
+// K of the GEMM is the position, which is the strided index of the
+// channels-last arrays.  ds_read_b64_tr_b16 transposes on the way out of LDS:
+// 16 lanes read 4 positions x 16 channels and lane r receives channel r of
+// the 4 positions, so two reads make the 8-position fragment of
+// v_mfma_f32_16x16x32_bf16.  Both operands use the same order of positions.
+// LDS rows are 16 channels (32 bytes), one block of rows per 16 channels: the
+// 16 rows of a read are then 512 contiguous bytes, without bank conflicts.
+//
+// A block's sums stay in registers over all its columns and are written
+// once; wgrad_reduce_kernel adds the blocks' sums in a fixed order.
+//
+// Bound by LDS reads and MFMAs alike: (7 + NF) fragments are read per 7 NF
+// MFMAs, so the array with more channels is the fixed one; NF is at most 5,
+// which is what 256 registers hold.  On 4 x 64^3, 80 -> 32 channels takes
+// 133 us (1.09 PFLOP/s), and the 12 layers of the network 0.52 ms with the
+// reductions, against 14.6 ms when every block staged its positions again
+// for each tap and transposed the fragments with 2-byte LDS reads.
 
-__global__ void __launch_bounds__(256)
-conv3_wgrad_kernel(const uint16_t * __restrict__ x, const uint16_t * __restrict__ dy,
-		   float * __restrict__ part, int64_t npos, int64_t chunk,
-		   int nx, int ny, int nz, int cin, int cout) {
-  __shared__ uint16_t sy[WG_P][WG_CMAX + 4];
-  __shared__ uint16_t sx[WG_P][WG_CMAX + 4];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int r = lane & 15, kq = lane >> 4;
-  const int t = blockIdx.y;
-  const int64_t pbeg = (int64_t) blockIdx.x*chunk;
-  const int64_t pend = (pbeg + chunk < npos) ? pbeg + chunk : npos;
-  const int nco = cout/16, nci = cin/16;
-  const int npair = nco*nci;
-  // this block's pairs: [16*blockIdx.z, 16*blockIdx.z + 16); wave: 4 of them
-  int pco[4], pci[4];
-  bool has[4];
-#pragma unroll
-  for (int j = 0; j < 4; j++) {
-    const int pr = 16*blockIdx.z + 4*wave + j;
-    has[j] = (pr < npair);
-    pco[j] = has[j] ? pr / nci : 0;
-    pci[j] = has[j] ? pr % nci : 0;
-  }
-  f4 acc[4];
-#pragma unroll
-  for (int j = 0; j < 4; j++) acc[j] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u4a __attribute__((ext_vector_type(4), aligned(8)));   // 16 bytes, 8-byte aligned
 
-  for (int64_t p0 = pbeg; p0 < pend; p0 += WG_P) {
-    // stage 64 rows of dy and of x shifted by tap t (4 channels per load)
-    const int ly = cout/4, lx = cin/4;
-    for (int i = threadIdx.x; i < WG_P*ly; i += 256) {
-      const int row = i / ly, c = 4*(i - row*ly);
-      const int64_t p = p0 + row;
-      uint64_t v = 0;
-      if (p < pend) v = *reinterpret_cast<const uint64_t *>(dy + p*cout + c);
-      *reinterpret_cast<uint64_t *>(&sy[row][c]) = v;
+constexpr int WT_Y = 8, WT_Z = 16;
+constexpr int WT_N = WT_Y*WT_Z;                       // positions of a tile plane
+constexpr int WH_Z = WT_Z + 2, WH_N = (WT_Y + 2)*WH_Z; // with the halo
+constexpr int WT_TAPS = 7;                            // taps per wave
+constexpr int WG_BLOCKS = 512;                        // blocks of a launch: two per CU
+constexpr int WG_NF_MAX = 5;
+
+struct WgradPlan {
+  int shift_x;                   // x is the shifted array (else dy)
+  int nf, nfg, ns;               // fixed 16-channel blocks per block, groups of them; shifted blocks
+  int ty, tz, xlen, xc;          // tiles in y and z, planes per item, items along x
+  int items, nchunk;             // (sample, column, x range) items; blocks that share them
+};
+
+WgradPlan wgrad_plan(int batch, int nx, int ny, int nz, int cin, int cout) {
+  WgradPlan w;
+  const int bi = cin/16, bo = cout/16;
+  w.shift_x = (cin <= cout);
+  w.ns = w.shift_x ? bi : bo;
+  const int f = w.shift_x ? bo : bi;
+  w.nfg = (f + WG_NF_MAX - 1)/WG_NF_MAX;
+  w.nf = (f + w.nfg - 1)/w.nfg;
+  w.ty = (ny + WT_Y - 1)/WT_Y;
+  w.tz = (nz + WT_Z - 1)/WT_Z;
+  const int cols = batch*w.ty*w.tz;
+  int want = WG_BLOCKS/(w.ns*w.nfg);
+  if (want < 1) want = 1;
+  // x ranges of at least 2 planes (each reads 2 halo planes more) until the
+  // items make the wanted number of blocks
+  int xc = (want + cols - 1)/cols;
+  if (xc > (nx + 1)/2) xc = (nx + 1)/2;
+  w.xlen = (nx + xc - 1)/xc;
+  w.xc = (nx + w.xlen - 1)/w.xlen;
+  w.items = cols*w.xc;
+  w.nchunk = (w.items < want) ? w.items : want;
+  return w;
+}
+
+__device__ __forceinline__ s4 read_tr(const uint16_t * p) {
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+    (__attribute__((address_space(3))) s4 *) const_cast<uint16_t *>(p));
+}
+
+__device__ __forceinline__ b8 join8(s4 lo, s4 hi) {
+  const s8 v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+  return __builtin_bit_cast(b8, v);
+}
+
+// fx, sx: the fixed and the shifted array, cf and cs channels
+template <int NF, bool SHIFT_X>
+__global__ void __launch_bounds__(256, 2)
+conv3_wgrad_kernel(const uint16_t * __restrict__ fx, const uint16_t * __restrict__ sx,
+		   float * __restrict__ part, int nx, int ny, int nz, int cf, int cs,
+		   int ty, int tz, int xlen, int xc, int items) {
+  __shared__ __attribute__((aligned(16))) uint16_t ls[4][WH_N*16];
+  __shared__ __attribute__((aligned(16))) uint16_t lf[2][NF][WT_N*16];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = tid >> 6;
+  const int r = lane & 15, q = lane >> 4;
+  const int s0 = 16*(blockIdx.y % (cs/16));              // first shifted channel
+  const int f0 = 16*NF*(blockIdx.y / (cs/16));           // first fixed channel
+
+  f4 acc[WT_TAPS][NF];
+#pragma unroll
+  for (int j = 0; j < WT_TAPS; j++)
+#pragma unroll
+    for (int k = 0; k < NF; k++) acc[j][k] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+
+  // this lane's part of a transposing read: position 4q + (r >> 2) of a row
+  // of 16, channels 4 (r & 3) .. + 3
+  const int lpos = 4*q + (r >> 2), lch = 4*(r & 3);
+  const int half = 8*(tid & 1);                          // staging: 8 channels per thread
+
+  for (int item = blockIdx.x; item < items; item += gridDim.x) {
+    int c = item;
+    const int xi = c % xc; c /= xc;
+    const int z0 = (c % tz)*WT_Z; c /= tz;
+    const int y0 = (c % ty)*WT_Y;
+    const int b = c / ty;
+    const int xb = xi*xlen;
+    const int n = min(xlen, nx - xb);                    // planes of this item
+    const int64_t plane = (int64_t) ny*nz;
+    const uint16_t * fb = fx + (int64_t) b*nx*plane*cf + f0 + half;
+    const uint16_t * sb = sx + (int64_t) b*nx*plane*cs + s0 + half;
+
+    // staging positions within a plane; -1: outside the lattice, staged as
+    // zeros (in the shifted tile everything past the wrapped halo)
+    const int fr = tid >> 1;
+    const int fy = y0 + fr/WT_Z, fz = z0 + fr%WT_Z;
+    const int64_t fo = (fy < ny && fz < nz) ? ((int64_t) fy*nz + fz)*cf : -1;
+    int64_t so[2];
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+      const int row = (tid + 256*k) >> 1;
+      const int y = y0 + row/WH_Z - 1, z = z0 + row%WH_Z - 1;
+      so[k] = (row < WH_N && y <= ny && z <= nz) ? ((int64_t) wrapi(y, ny)*nz + wrapi(z, nz))*cs : -1;
     }
-    for (int i = threadIdx.x; i < WG_P*lx; i += 256) {
-      const int row = i / lx, c = 4*(i - row*lx);
-      const int64_t p = p0 + row;
-      uint64_t v = 0;
-      if (p < pend) {
-	const Pos q = pos_of(p, nx, ny, nz);
-	v = *reinterpret_cast<const uint64_t *>(x + shifted(q, t, nx, ny, nz)*cin + c);
+    u4 rf[NF], rs[2];
+    auto fetch_f = [&](int x) {
+#pragma unroll
+      for (int k = 0; k < NF; k++) {
+	rf[k] = u4{0u, 0u, 0u, 0u};
+	if (fo >= 0 && f0 + 16*k < cf) rf[k] = *reinterpret_cast<const u4a *>(fb + x*plane*cf + fo + 16*k);
       }
-      *reinterpret_cast<uint64_t *>(&sx[row][c]) = v;
-    }
+    };
+    auto fetch_s = [&](int x) {
+      const int xw = wrapi(x, nx);
+#pragma unroll
+      for (int k = 0; k < 2; k++) {
+	rs[k] = u4{0u, 0u, 0u, 0u};
+	if (so[k] >= 0) rs[k] = *reinterpret_cast<const u4a *>(sb + xw*plane*cs + so[k]);
+      }
+    };
+    auto store_f = [&](int i) {
+#pragma unroll
+      for (int k = 0; k < NF; k++) *reinterpret_cast<u4 *>(&lf[i & 1][k][8*tid]) = rf[k];
+    };
+    auto store_s = [&](int i) {
+#pragma unroll
+      for (int k = 0; k < 2; k++)
+	if (tid + 256*k < 2*WH_N) *reinterpret_cast<u4 *>(&ls[i & 3][8*(tid + 256*k)]) = rs[k];
+    };
+
+    // shifted plane xb - 1 + i sits in slot i & 3, fixed plane xb + i in i & 1
+    fetch_s(xb - 1); store_s(0);
+    fetch_s(xb); store_s(1);
+    fetch_s(xb + 1); store_s(2);
+    fetch_f(xb); store_f(0);
     __syncthreads();
+#pragma unroll 1
+    for (int i = 0; i < n; i++) {
+      const bool more = (i + 1 < n);
+      if (more) { fetch_s(xb + i + 2); fetch_f(xb + i + 1); }
+      const uint16_t * pf = &lf[i & 1][0][lpos*16 + lch];
+      const uint16_t * ps[WT_TAPS];
 #pragma unroll
-    for (int ks = 0; ks < WG_P/16; ks++) {
+      for (int j = 0; j < WT_TAPS; j++) {
+	const int t = min(WT_TAPS*wave + j, 26);
+	const int dx = t/9, dy = (t/3)%3, dz = t%3;
+	ps[j] = &ls[(i + dx) & 3][(dy*WH_Z + dz + lpos)*16 + lch];
+      }
+#pragma unroll 1
+      for (int ks = 0; ks < WT_Y/2; ks++) {
+	b8 ff[NF];
 #pragma unroll
-      for (int j = 0; j < 4; j++) {
-	if (!has[j]) continue;
-	s4 a, b;
+	for (int k = 0; k < NF; k++)
+	  ff[k] = join8(read_tr(pf + (k*WT_N + 2*ks*WT_Z)*16), read_tr(pf + (k*WT_N + (2*ks + 1)*WT_Z)*16));
 #pragma unroll
-	for (int i = 0; i < 4; i++) {
-	  a[i] = (short) sy[16*ks + 4*kq + i][16*pco[j] + r];
-	  b[i] = (short) sx[16*ks + 4*kq + i][16*pci[j] + r];
+	for (int j = 0; j < WT_TAPS; j++) {
+	  const b8 sf = join8(read_tr(ps[j] + 2*ks*WH_Z*16), read_tr(ps[j] + (2*ks + 1)*WH_Z*16));
+#pragma unroll
+	  for (int k = 0; k < NF; k++)
+	    acc[j][k] = SHIFT_X ? __builtin_amdgcn_mfma_f32_16x16x32_bf16(ff[k], sf, acc[j][k], 0, 0, 0)
+				: __builtin_amdgcn_mfma_f32_16x16x32_bf16(sf, ff[k], acc[j][k], 0, 0, 0);
 	}
-	acc[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[j], 0, 0, 0);
       }
+      // the slots written here were last read one plane ago
+      if (more) { store_s(i + 3); store_f(i + 1); }
+      __syncthreads();
     }
-    __syncthreads();
   }
-  // partial[chunk][t][co][ci]
+
+  // part[block][t][co][ci]; D: lane holds rows (co) 4q + i of column (ci) r
+  const int cin = SHIFT_X ? cs : cf, cout = SHIFT_X ? cf : cs;
 #pragma unroll
-  for (int j = 0; j < 4; j++) {
-    if (!has[j]) continue;
+  for (int j = 0; j < WT_TAPS; j++) {
+    const int st = WT_TAPS*wave + j;
+    if (st >= 27) continue;
+    const int t = SHIFT_X ? st : 26 - st;
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int co = 16*pco[j] + 4*kq + i, ci = 16*pci[j] + r;
-      part[(((int64_t) blockIdx.x*27 + t)*cout + co)*cin + ci] = acc[j][i];
+    for (int k = 0; k < NF; k++) {
+      if (f0 + 16*k >= cf) continue;
+      const int co = (SHIFT_X ? f0 + 16*k : s0) + 4*q, ci = (SHIFT_X ? s0 : f0 + 16*k) + r;
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+	part[(((int64_t) blockIdx.x*27 + t)*cout + co + i)*cin + ci] = acc[j][k][i];
     }
   }
 }
 
-__global__ void wgrad_reduce_kernel(const float * __restrict__ part, float * __restrict__ dw,
-				    int nchunk, int64_t n, int accumulate) {
-  for (int64_t i = blockIdx.x*(int64_t) blockDim.x + threadIdx.x; i < n; i += (int64_t) gridDim.x*blockDim.x) {
-    float s = 0.0f;
-    for (int c = 0; c < nchunk; c++) s += part[(int64_t) c*n + i];
-    dw[i] = accumulate ? dw[i] + s : s;
+// dw[i] (+)= sum over the blocks of part[block][i]: 64 values per block, the
+// four waves take every fourth partial and their sums are added in order
+__global__ void __launch_bounds__(256)
+wgrad_reduce_kernel(const float * __restrict__ part, float * __restrict__ dw, int nchunk, int64_t n,
+		    int accumulate) {
+  __shared__ float sh[4][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t i = (int64_t) blockIdx.x*64 + lane;
+  float s = 0.0f;
+  if (i < n) {
+#pragma unroll 8
+    for (int c = wave; c < nchunk; c += 4) s += part[(int64_t) c*n + i];
+  }
+  sh[wave][lane] = s;
+  __syncthreads();
+  if (wave == 0 && i < n) {
+    const float v = (sh[0][lane] + sh[1][lane]) + (sh[2][lane] + sh[3][lane]);
+    dw[i] = accumulate ? dw[i] + v : v;
   }
 }
 
@@ -683,33 +828,32 @@ hipError_t launch_conv3_fwd(const uint16_t * x, const uint16_t * w, const float 
   return hipGetLastError();
 }
 
-int64_t conv3_wgrad_workspace(int batch, int nx, int ny, int nz, int cin, int cout, int * nchunk,
-			      int64_t * chunk) {
-  const int64_t npos = (int64_t) batch*nx*ny*nz;
-  const int groups = (cout/16*(cin/16) + 15)/16;
-  // about 2048 blocks in all; chunks are whole 64-position slices
-  int64_t nc = 2048/(27*groups);
-  if (nc < 1) nc = 1;
-  int64_t ch = (npos + nc - 1)/nc;
-  ch = ((ch + WG_P - 1)/WG_P)*WG_P;
-  nc = (npos + ch - 1)/ch;
-  *nchunk = (int) nc;
-  *chunk = ch;
-  return nc*27*(int64_t) cout*cin;
+int64_t conv3_wgrad_workspace(int batch, int nx, int ny, int nz, int cin, int cout) {
+  return (int64_t) wgrad_plan(batch, nx, ny, nz, cin, cout).nchunk*27*cout*cin;
 }
 
 hipError_t launch_conv3_wgrad(const uint16_t * x, const uint16_t * dy, float * dw, float * work,
 			      int batch, int nx, int ny, int nz, int cin, int cout, int accumulate,
 			      hipStream_t s) {
-  int nchunk;
-  int64_t chunk;
-  conv3_wgrad_workspace(batch, nx, ny, nz, cin, cout, &nchunk, &chunk);
-  const int64_t npos = (int64_t) batch*nx*ny*nz;
-  const int groups = (cout/16*(cin/16) + 15)/16;
-  hipLaunchKernelGGL(conv3_wgrad_kernel, dim3(nchunk, 27, groups), dim3(256), 0, s,
-		     x, dy, work, npos, chunk, nx, ny, nz, cin, cout);
+  const WgradPlan w = wgrad_plan(batch, nx, ny, nz, cin, cout);
+  const dim3 grid(w.nchunk, w.ns*w.nfg), block(256);
+#define WG_(NF) do { \
+    if (w.shift_x) hipLaunchKernelGGL((conv3_wgrad_kernel<NF, true>), grid, block, 0, s, dy, x, work, nx, ny, nz, \
+				      cout, cin, w.ty, w.tz, w.xlen, w.xc, w.items); \
+    else hipLaunchKernelGGL((conv3_wgrad_kernel<NF, false>), grid, block, 0, s, x, dy, work, nx, ny, nz, \
+			    cin, cout, w.ty, w.tz, w.xlen, w.xc, w.items); \
+  } while (0)
+  switch (w.nf) {
+  case 1: WG_(1); break;
+  case 2: WG_(2); break;
+  case 3: WG_(3); break;
+  case 4: WG_(4); break;
+  default: WG_(5); break;
+  }
+#undef WG_
   const int64_t n = (int64_t) 27*cout*cin;
-  hipLaunchKernelGGL(wgrad_reduce_kernel, dim3(grid_for(n)), dim3(256), 0, s, work, dw, nchunk, n, accumulate);
+  hipLaunchKernelGGL(wgrad_reduce_kernel, dim3((unsigned) ((n + 63)/64)), dim3(256), 0, s, work, dw, w.nchunk, n,
+		     accumulate);
   return hipGetLastError();
 }
 

@@ -183,8 +183,7 @@ hipError_t launch_conv3_fwd(const uint16_t * x, const uint16_t * w, const float 
 			    uint16_t * act, int batch, int nx, int ny, int nz, int cin, int cout,
 			    int accumulate, hipStream_t s);
 // floats of workspace for launch_conv3_wgrad
-int64_t conv3_wgrad_workspace(int batch, int nx, int ny, int nz, int cin, int cout, int * nchunk,
-			      int64_t * chunk);
+int64_t conv3_wgrad_workspace(int batch, int nx, int ny, int nz, int cin, int cout);
 hipError_t launch_conv3_wgrad(const uint16_t * x, const uint16_t * dy, float * dw, float * work,
 			      int batch, int nx, int ny, int nz, int cin, int cout, int accumulate,
 			      hipStream_t s);

@@ -116,9 +116,7 @@ extern "C" int ldw_conv3d_bwd_weight(const void * x, const void * dy, float * dw
   READY();
   if (check_conv(batch, nx, ny, nz, cin, cout)) return -1;
   if (cin > 160 || cout > 160) LDW_FAIL("conv3d weight gradient: at most 160 channels (cin %d, cout %d)", cin, cout);
-  int nchunk;
-  int64_t chunk;
-  const int64_t n = ldw::conv3_wgrad_workspace(batch, nx, ny, nz, cin, cout, &nchunk, &chunk);
+  const int64_t n = ldw::conv3_wgrad_workspace(batch, nx, ny, nz, cin, cout);
   void * work = nullptr;
   if (scratch_buffer(g_wgrad, (size_t) n*sizeof(float), &work)) return -1;
   KCHECK(ldw::launch_conv3_wgrad((const uint16_t *) x, (const uint16_t *) dy, dw, (float *) work, batch,

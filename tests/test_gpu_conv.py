@@ -96,6 +96,31 @@ def test_conv_fwd_bwd_against_oracle(cin, cout, batch, shape):
     within(y.download().astype(np.float64), 2 * yo, 4 * 27 * cin * EPS32 * ya + 1e-30, "forward x2")
 
 
+# the weight gradient's tiles are 8 x 16 (y, z) columns marched along x: one
+# site, ragged tiles on both sides of an edge, single planes, uneven x ranges,
+# either operand shifted, one to ten 16-channel blocks of the fixed operand
+# (odd counts leave half-filled groups), and more columns than blocks
+@pytest.mark.parametrize("cin,cout,batch,shape", [
+    (16, 16, 1, (1, 1, 1)), (16, 48, 2, (2, 7, 15)), (48, 16, 1, (3, 8, 16)), (32, 64, 1, (1, 9, 17)),
+    (80, 16, 2, (5, 1, 33)), (16, 96, 1, (9, 17, 5)), (112, 32, 1, (3, 16, 32)), (64, 160, 1, (2, 9, 18)),
+    (96, 96, 2, (2, 40, 80))])
+@pytest.mark.parametrize("accumulate", [0, 1])
+def test_conv_weight_gradient_tiles(cin, cout, batch, shape, accumulate):
+    lib = L.lib()
+    rng = np.random.default_rng(7 * cin + cout + shape[1])
+    n = batch * int(np.prod(shape))
+    x, g = bf16_round(rng.standard_normal(n * cin)), bf16_round(rng.standard_normal(n * cout))
+    before = rng.standard_normal(27 * cout * cin).astype(np.float32)
+    dx, dg, dw = dev(bf16_bits(x), np.uint16), dev(bf16_bits(g), np.uint16), dev(before, np.float32)
+    print(f"weight gradient cin={cin} cout={cout} batch={batch} shape={shape}", flush=True)
+    assert lib.ldw_conv3d_bwd_weight(vp(dx), vp(dg), vp(dw), batch, *shape, cin, cout, accumulate) == 0
+    want = O.conv3_bwd_weight(x, g, shape, cin, cout, batch)
+    mag = O.conv3_bwd_weight(np.abs(x), np.abs(g), shape, cin, cout, batch)
+    if accumulate:
+        want, mag = want + before, mag + np.abs(before)
+    within(dw.download().astype(np.float64), want, 2 * (n + 1) * EPS32 * mag + 1e-30, "weight gradient")
+
+
 def test_pool_up_concat_split_silu_exact():
     lib = L.lib()
     rng = np.random.default_rng(1)
