@@ -42,34 +42,103 @@ __global__ void silu_fwd_kernel(const float * __restrict__ z, uint16_t * __restr
 }
 
 // dz = da sigma(z) (1 + z (1 - sigma(z)))
+__device__ __forceinline__ float silu_grad(float v, float da) {
+  const float s = 1.0f/(1.0f + expf(-v));
+  return da*s*(1.0f + v*(1.0f - s));
+}
+
 __global__ void silu_bwd_kernel(const float * __restrict__ z, const float * __restrict__ da,
 				float * __restrict__ dz, uint16_t * __restrict__ dzb, int64_t n) {
   GRID_STRIDE(i, n) {
-    const float v = z[i];
-    const float s = 1.0f/(1.0f + expf(-v));
-    const float g = da[i]*s*(1.0f + v*(1.0f - s));
+    const float g = silu_grad(z[i], da[i]);
     if (dz) dz[i] = g;
     dzb[i] = bf16_of(g);
   }
 }
 
-// per-block partial sums of each channel over a slice of positions
-__global__ void bias_grad_kernel(const float * __restrict__ dz, float * __restrict__ part,
-				 int64_t npos, int c, int64_t chunk) {
-  const int64_t p0 = blockIdx.x*chunk;
-  const int64_t p1 = (p0 + chunk < npos) ? p0 + chunk : npos;
-  for (int ch = threadIdx.x; ch < c; ch += blockDim.x) {
-    float s = 0.0f;
-    for (int64_t p = p0; p < p1; p++) s += dz[p*c + ch];
-    part[(int64_t) blockIdx.x*c + ch] = s;
+__device__ __forceinline__ uint2 bf16x4(const float4 & g) {
+  return make_uint2(bf16_of(g.x) | ((uint32_t) bf16_of(g.y) << 16), bf16_of(g.z) | ((uint32_t) bf16_of(g.w) << 16));
+}
+
+// the same, 4 values per thread, for n a multiple of 4 and arrays aligned
+// for it: bound by memory (15.8 M values, 14 bytes each: 40 -> 35 us)
+__global__ void silu_bwd4_kernel(const float4 * __restrict__ z, const float4 * __restrict__ da,
+				 float4 * __restrict__ dz, uint2 * __restrict__ dzb, int64_t n4) {
+  GRID_STRIDE(i, n4) {
+    const float4 v = z[i], d = da[i];
+    const float4 g = make_float4(silu_grad(v.x, d.x), silu_grad(v.y, d.y), silu_grad(v.z, d.z), silu_grad(v.w, d.w));
+    if (dz) dz[i] = g;
+    dzb[i] = bf16x4(g);
   }
 }
 
-__global__ void sum_rows_kernel(const float * __restrict__ part, float * __restrict__ out,
-				int nrow, int c, int accumulate) {
-  for (int ch = blockIdx.x*blockDim.x + threadIdx.x; ch < c; ch += gridDim.x*blockDim.x) {
-    float s = 0.0f;
-    for (int r = 0; r < nrow; r++) s += part[(int64_t) r*c + ch];
+// Sums of each channel over the positions, in two passes: partial sums of
+// SUM_ROWS blocks, then their sums in a fixed order.
+//
+// A block's threads cover `rows` whole positions at a time, V channels each,
+// so its loads are contiguous whatever the channel count; the last channels
+// of a wide array go to further blocks in y.  Bound by reading dz: 32
+// channels at 2^20 positions take 30 us (4.5 TB/s), the sums of the partial
+// rows 5 us.  With one thread per channel walking its positions and one
+// summing the partials, the 12 layers of a 4 x 64^3 training step took 4.2 ms
+// (now 0.22 ms).
+constexpr int SUM_ROWS = 1024;
+
+template <int V>
+__global__ void __launch_bounds__(256)
+bias_grad_kernel(const float * __restrict__ dz, float * __restrict__ part, int64_t npos, int c) {
+  __shared__ float sh[256*V];
+  const int cv = c/V;                               // columns of V channels
+  const int tr = (cv < 256) ? cv : 256;             // threads per position
+  const int rows = 256/tr;
+  const int row = threadIdx.x/tr, col = blockIdx.y*256 + threadIdx.x%tr;
+  const bool has = (row < rows && col < cv);
+  float s[V];
+#pragma unroll
+  for (int k = 0; k < V; k++) s[k] = 0.0f;
+  if (has) {
+    const float * a = dz + (int64_t) V*col;
+#pragma unroll 4
+    for (int64_t p = (int64_t) blockIdx.x*rows + row; p < npos; p += (int64_t) gridDim.x*rows) {
+      if constexpr (V == 4) {
+	const float4 v = *reinterpret_cast<const float4 *>(a + p*c);
+	s[0] += v.x; s[1] += v.y; s[2] += v.z; s[3] += v.w;
+      }
+      else {
+	s[0] += a[p*c];
+      }
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < V; k++) sh[V*threadIdx.x + k] = s[k];
+  __syncthreads();
+  if (row == 0 && has) {
+#pragma unroll
+    for (int k = 0; k < V; k++) {
+      float t = s[k];
+      for (int j = 1; j < rows; j++) t += sh[V*(threadIdx.x + j*tr) + k];
+      part[(int64_t) blockIdx.x*c + V*col + k] = t;
+    }
+  }
+}
+
+// out[ch] (+)= sum over the rows of part[row][ch], in a fixed order: a block
+// sums up to 64 channels, its slices of threads every slices-th row
+__global__ void __launch_bounds__(1024)
+sum_rows_kernel(const float * __restrict__ part, float * __restrict__ out, int nrow, int c, int accumulate) {
+  __shared__ float sh[1024];
+  const int cc = (c < 64) ? c : 64;
+  const int slices = 1024/cc;
+  const int slice = threadIdx.x/cc, ch = blockIdx.x*cc + threadIdx.x%cc;
+  float s = 0.0f;
+  if (slice < slices && ch < c) {
+#pragma unroll 8
+    for (int r = slice; r < nrow; r += slices) s += part[(int64_t) r*c + ch];
+  }
+  sh[threadIdx.x] = s;
+  __syncthreads();
+  if (slice == 0 && ch < c) {
+    for (int k = 1; k < slices; k++) s += sh[threadIdx.x + k*cc];
     out[ch] = accumulate ? out[ch] + s : s;
   }
 }
@@ -400,10 +469,16 @@ __global__ void plane_shift_kernel(float * __restrict__ out, int64_t ns, int npl
        i += (int64_t) gridDim.x*blockDim.x) a[i] += d;
 }
 
+// one wave: every lane adds each 64th partial, lane 0 the lanes' sums (a
+// serial sum of 512 partials waited for each load in turn, 35 us against 4)
 __global__ void sum_parts_kernel(const double * __restrict__ part, int nb, double * __restrict__ out) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    double s = 0.0;
-    for (int b = 0; b < nb; b++) s += part[b];
+  __shared__ double sh[64];
+  double s = 0.0;
+  for (int b = threadIdx.x; b < nb; b += 64) s += part[b];
+  sh[threadIdx.x] = s;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int k = 1; k < 64; k++) s += sh[k];
     out[0] = s;
   }
 }
@@ -419,24 +494,39 @@ hipError_t nn_silu_fwd(const float * z, uint16_t * a, int64_t n, hipStream_t s) 
 
 hipError_t nn_silu_bwd(const float * z, const float * da, float * dz, uint16_t * dzb, int64_t n,
 		       hipStream_t s) {
-  LAUNCH(silu_bwd_kernel, n, z, da, dz, dzb, n);
+  if (n % 4 == 0 && (((uintptr_t) z | (uintptr_t) da | (uintptr_t) dz) % 16) == 0 && ((uintptr_t) dzb % 8) == 0) {
+    LAUNCH(silu_bwd4_kernel, n/4, reinterpret_cast<const float4 *>(z), reinterpret_cast<const float4 *>(da),
+	   reinterpret_cast<float4 *>(dz), reinterpret_cast<uint2 *>(dzb), n/4);
+  }
+  else {
+    LAUNCH(silu_bwd_kernel, n, z, da, dz, dzb, n);
+  }
   return hipGetLastError();
 }
 
 int64_t nn_bias_grad_workspace(int64_t npos, int c) {
   (void) npos;
-  return (int64_t) 1024*c;
+  return (int64_t) SUM_ROWS*c;
+}
+
+void launch_sum_rows(const float * part, float * out, int nrow, int c, int accumulate, hipStream_t s) {
+  const int cc = (c < 64) ? c : 64;
+  hipLaunchKernelGGL(sum_rows_kernel, dim3((c + cc - 1)/cc), dim3(1024), 0, s, part, out, nrow, c, accumulate);
 }
 
 hipError_t nn_bias_grad(const float * dz, float * db, float * work, int64_t npos, int c,
 			int accumulate, hipStream_t s) {
-  int64_t nblk = 1024;
-  if (npos < nblk) nblk = npos > 0 ? npos : 1;
-  const int64_t chunk = (npos + nblk - 1)/nblk;
-  nblk = (npos + chunk - 1)/chunk;
+  const bool v4 = (c % 4 == 0 && ((uintptr_t) dz % 16) == 0);
+  const int cv = v4 ? c/4 : c;
+  const int rows = (cv < 256) ? 256/cv : 1;
+  // no more blocks than have a position
+  int64_t nblk = (npos + rows - 1)/rows;
   if (nblk < 1) nblk = 1;
-  hipLaunchKernelGGL(bias_grad_kernel, dim3((unsigned) nblk), dim3(64), 0, s, dz, work, npos, c, chunk);
-  hipLaunchKernelGGL(sum_rows_kernel, dim3((c + 255)/256), dim3(256), 0, s, work, db, (int) nblk, c, accumulate);
+  if (nblk > SUM_ROWS) nblk = SUM_ROWS;
+  const dim3 grid((unsigned) nblk, (cv + 255)/256);
+  if (v4) hipLaunchKernelGGL(bias_grad_kernel<4>, grid, dim3(256), 0, s, dz, work, npos, c);
+  else hipLaunchKernelGGL(bias_grad_kernel<1>, grid, dim3(256), 0, s, dz, work, npos, c);
+  launch_sum_rows(work, db, (int) nblk, c, accumulate, s);
   return hipGetLastError();
 }
 

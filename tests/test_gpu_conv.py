@@ -121,6 +121,47 @@ def test_conv_weight_gradient_tiles(cin, cout, batch, shape, accumulate):
     within(dw.download().astype(np.float64), want, 2 * (n + 1) * EPS32 * mag + 1e-30, "weight gradient")
 
 
+def at(d, nbytes):
+    """The device address nbytes into d."""
+    return ctypes.c_void_p(d.ptr + nbytes)
+
+
+# channel counts below, at and above what a block's 256 threads cover, 4 at a
+# time or singly, positions fewer and more than the blocks; off = 1 shifts the
+# array off 16-byte alignment
+@pytest.mark.parametrize("c", [1, 3, 16, 48, 100, 260, 1028])
+@pytest.mark.parametrize("npos", [1, 70, 5003])
+@pytest.mark.parametrize("off", [0, 1])
+def test_bias_gradient_shapes(c, npos, off):
+    lib = L.lib()
+    rng = np.random.default_rng(c + npos)
+    a = rng.standard_normal(npos * c + off).astype(np.float32)
+    d, db = dev(a, np.float32), dev(np.ones(c, np.float32), np.float32)
+    v = a[off:].reshape(npos, c).astype(np.float64)
+    for acc in (0, 1):
+        assert lib.ldw_nn_bias_grad(at(d, 4 * off), vp(db), npos, c, acc) == 0
+        want = (1 + acc) * v.sum(0)
+        within(db.download().astype(np.float64), want, 2 * (npos + 2) * EPS32 * 2 * np.abs(v).sum(0) + 1e-30, "bias")
+
+
+@pytest.mark.parametrize("n", [1, 4, 1003, 4096])
+def test_silu_backward_vector_path_is_the_scalar_one(n):
+    lib = L.lib()
+    rng = np.random.default_rng(n)
+    z, da = (4 * rng.standard_normal(n)).astype(np.float32), rng.standard_normal(n).astype(np.float32)
+    out = []
+    for off in (0, 1):
+        pad = np.zeros(off, np.float32)
+        dz_, dd = dev(np.concatenate([pad, z]), np.float32), dev(np.concatenate([pad, da]), np.float32)
+        g, gb = L.DeviceArray(n + off, np.float32), L.DeviceArray(n + off, np.uint16)
+        assert lib.ldw_nn_silu_bwd(at(dz_, 4 * off), at(dd, 4 * off), at(g, 4 * off), at(gb, 2 * off), n) == 0
+        out.append((g.download()[off:], gb.download()[off:]))
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+    zz = z.astype(np.float64)
+    sg = 1 / (1 + np.exp(-zz))
+    assert np.allclose(out[0][0], da * sg * (1 + zz * (1 - sg)), rtol=1e-5, atol=1e-6)
+
+
 def test_pool_up_concat_split_silu_exact():
     lib = L.lib()
     rng = np.random.default_rng(1)
