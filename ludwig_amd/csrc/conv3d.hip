@@ -8,12 +8,9 @@
 // and the adjoint of a convolution is again a convolution.  Channel
 // counts are multiples of 16.
 //
-// Forward, y = b + sum_t W_t x(p + o_t):  GEMM with M = positions,
-//   N = Cout, K = 27 Cin.  A wave owns 32 positions x 16*NT16 output
-//   channels: 2 x NT16 tiles of v_mfma_f32_16x16x16_bf16.  The A fragment
-//   of a lane is 4 consecutive channels of one (shifted) position and the
-//   B fragment 4 consecutive input channels of one output channel, so both
-//   are single 8-byte loads with weights stored as W[t][cout][cin].
+// Forward, y = b + sum_t W_t x(p + o_t):  GEMM with M = Cout, N = positions,
+//   K = 27 Cin; tiles of x with their halo are staged in LDS 16 channels at a
+//   time, each read for up to 3 taps.
 // Backward data, dx = sum_t W_{26-t}^T dy(p + o_t): the same kernel with the
 //   weights flipped and transposed (conv3_weights_prep).
 // Backward weight, dW_t = sum_p dy(p) x(p + o_t)^T:  GEMM with M = Cout,
@@ -23,9 +20,9 @@
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
-#include <stdlib.h>
 
 #include "kernels.h"
+#include "silu.h"
 
 namespace ldw {
 
@@ -38,446 +35,307 @@ __device__ __forceinline__ int wrapi(int i, int n) {
   return (i < 0) ? i + n : (i >= n ? i - n : i);
 }
 
-struct Pos { int b, x, y, z; };
-
-__device__ __forceinline__ uint16_t silu_bf16(float v) {
-  uint32_t u = __float_as_uint(v/(1.0f + expf(-v)));
-  if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t) ((u >> 16) | 0x40u);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return (uint16_t) (u >> 16);
-}
-
-// epilogue: y = acc + bias (+ y) if y is given; a = bf16(SiLU(that)) if a is given
-__device__ __forceinline__ void store_out(float * __restrict__ y, uint16_t * __restrict__ a, int64_t idx,
-					  float v, int accumulate) {
-  if (y) {
-    if (accumulate) v += y[idx];
-    y[idx] = v;
-  }
-  if (a) a[idx] = silu_bf16(v);
-}
-
-__device__ __forceinline__ Pos pos_of(int64_t p, int nx, int ny, int nz) {
-  Pos q;
-  q.z = (int) (p % nz); p /= nz;
-  q.y = (int) (p % ny); p /= ny;
-  q.x = (int) (p % nx); p /= nx;
-  q.b = (int) p;
-  return q;
-}
-
-__device__ __forceinline__ int64_t shifted(const Pos & q, int t, int nx, int ny, int nz) {
-  const int dx = t/9 - 1, dy = (t/3)%3 - 1, dz = t%3 - 1;
-  return (((int64_t) q.b*nx + wrapi(q.x + dx, nx))*ny + wrapi(q.y + dy, ny))*nz + wrapi(q.z + dz, nz);
-}
-
-template <int NT16>
-__global__ void __launch_bounds__(256)
-conv3_fwd_kernel(const uint16_t * __restrict__ x, const uint16_t * __restrict__ w,
-		 const float * __restrict__ bias, float * __restrict__ y, uint16_t * __restrict__ act,
-		 int64_t npos, int nx, int ny, int nz, int cin, int cout, int accumulate) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int r = lane & 15, kq = lane >> 4;
-  const int64_t m0 = (int64_t) blockIdx.x*(blockDim.x/2) + wave*32;   // 32 positions per wave
-  const int n0 = blockIdx.y*16*NT16;
-
-  Pos q[2];
-  bool ok[2];
-#pragma unroll
-  for (int rb = 0; rb < 2; rb++) {
-    const int64_t p = m0 + 16*rb + r;
-    ok[rb] = (p < npos);
-    q[rb] = pos_of(ok[rb] ? p : 0, nx, ny, nz);
-  }
-  f4 acc[2][NT16];
-#pragma unroll
-  for (int rb = 0; rb < 2; rb++)
-#pragma unroll
-    for (int nb = 0; nb < NT16; nb++) acc[rb][nb] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-
-  for (int t = 0; t < 27; t++) {
-    const int64_t s0 = shifted(q[0], t, nx, ny, nz)*cin + 4*kq;
-    const int64_t s1 = shifted(q[1], t, nx, ny, nz)*cin + 4*kq;
-    const uint16_t * wt = w + ((int64_t) t*cout + n0 + r)*cin + 4*kq;
-    for (int c0 = 0; c0 < cin; c0 += 16) {
-      s4 a0 = ok[0] ? *reinterpret_cast<const s4 *>(x + s0 + c0) : s4{0, 0, 0, 0};
-      s4 a1 = ok[1] ? *reinterpret_cast<const s4 *>(x + s1 + c0) : s4{0, 0, 0, 0};
-#pragma unroll
-      for (int nb = 0; nb < NT16; nb++) {
-	const s4 b = *reinterpret_cast<const s4 *>(wt + (int64_t) 16*nb*cin + c0);
-	acc[0][nb] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a0, b, acc[0][nb], 0, 0, 0);
-	acc[1][nb] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a1, b, acc[1][nb], 0, 0, 0);
-      }
-    }
-  }
-  // D layout: lane holds rows 4*kq + i of column r
-#pragma unroll
-  for (int rb = 0; rb < 2; rb++)
-#pragma unroll
-    for (int nb = 0; nb < NT16; nb++) {
-      const int ch = n0 + 16*nb + r;
-      const float bv = bias ? bias[ch] : 0.0f;
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-	const int64_t p = m0 + 16*rb + 4*kq + i;
-	if (p < npos) store_out(y, act, p*cout + ch, acc[rb][nb][i] + bv, accumulate);
-      }
-    }
-}
-
-// ---------------------------------------------------------------------------
-// LDS-tiled forward pass for lattices at least one tile in size.
-//
-// A block owns a 4 x 4 x 16 (x, y, z) tile of one sample and 16*NT output
-// channels; wave w owns the 4 z rows (x0 + w, y0 + j, z0..z0+15), j < 4,
-// i.e. 4 row blocks of 16 positions.  Input channels go in chunks of 32:
-// the chunk's 6 x 6 x 18 halo tile is staged in LDS once (periodic wrap on
-// load), so the 27 taps read their A fragments from LDS instead of
-// re-fetching them; the weights of 3 taps at a time are staged in LDS too,
-// shared by the 4 waves, and the next 3 taps' weights are fetched into
-// registers while the current ones are used.  v_mfma_f32_16x16x32_bf16:
-// a lane's A fragment is 8 consecutive channels of one position (16 bytes),
-// its B fragment 8 consecutive input channels of one output channel.
-
 typedef short s8 __attribute__((ext_vector_type(8)));
 typedef __bf16 b8 __attribute__((ext_vector_type(8)));
-
-constexpr int LT_X = 4, LT_Y = 4, LT_Z = 16;
-constexpr int LH_X = LT_X + 2, LH_Y = LT_Y + 2, LH_Z = LT_Z + 2;
-constexpr int LH_N = LH_X*LH_Y*LH_Z;          // 648 halo positions
-constexpr int LK = 32;                        // input channels per chunk
-constexpr int LNT_MAX = 6;                    // output channel blocks per block
-
-// LDS rows are 4 x 16 bytes (32 channels).  The 16 lanes of a fragment
-// read 16 consecutive rows at one 16-byte part, 64 bytes apart, which puts
-// them on the same banks; the part index is XOR-swizzled with bits of the
-// row index so that they spread over all banks.  swz_shift selects the bits.
-__device__ __forceinline__ int lds_part(int row, int part, int swz_shift) {
-  return part ^ ((row >> swz_shift) & 3);
-}
-
-template <int NT>
-__global__ void __launch_bounds__(256)
-conv3_fwd_lds_kernel(const uint16_t * __restrict__ x, const uint16_t * __restrict__ w,
-		     const float * __restrict__ bias, float * __restrict__ y, uint16_t * __restrict__ act,
-		     int nx, int ny, int nz, int cin, int cout, int accumulate,
-		     int ntx, int nty, int ntz, int swz) {
-  __shared__ uint4 sa[LH_N*(LK/8)];           // halo tile: [pos][4 x 8 channels]   41.5 KB
-  __shared__ uint4 sb[3][16*NT][LK/8];        // 3 taps x 16 NT outputs x 32 inputs
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int r = lane & 15, q = lane >> 4;
-  int t = blockIdx.x;
-  const int tz = t % ntz; t /= ntz;
-  const int ty = t % nty; t /= nty;
-  const int tx = t % ntx;
-  const int b = t / ntx;
-  const int x0 = tx*LT_X, y0 = ty*LT_Y, z0 = tz*LT_Z;
-  const int n0 = blockIdx.y*16*NT;
-  constexpr int NB = 3*16*NT*(LK/8);           // uint4 per weight stage
-  constexpr int NBT = (NB + 255)/256;          // per thread
-
-  f4 acc[4][NT];
-#pragma unroll
-  for (int j = 0; j < 4; j++)
-#pragma unroll
-    for (int n = 0; n < NT; n++) acc[j][n] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-
-  for (int c0 = 0; c0 < cin; c0 += LK) {
-    const int kc = (cin - c0 < LK) ? cin - c0 : LK;          // 16 or 32
-    for (int i = threadIdx.x; i < LH_N*4; i += 256) {
-      const int h = i >> 2, part = i & 3;
-      const int hz = h % LH_Z, hy = (h / LH_Z) % LH_Y, hx = h / (LH_Z*LH_Y);
-      uint4 v = {0u, 0u, 0u, 0u};
-      if (8*part < kc) {
-	const int gx = wrapi(x0 + hx - 1, nx), gy = wrapi(y0 + hy - 1, ny), gz = wrapi(z0 + hz - 1, nz);
-	v = *reinterpret_cast<const uint4 *>(x + ((((int64_t) b*nx + gx)*ny + gy)*nz + gz)*cin + c0 + 8*part);
-      }
-      sa[4*h + lds_part(h, part, swz)] = v;
-    }
-    // weights of taps 3s .. 3s+2: [tap][n][part]
-    uint4 pre[NBT];
-    auto fetch = [&](int st) {
-#pragma unroll
-      for (int k = 0; k < NBT; k++) {
-	const int i = threadIdx.x + 256*k;
-	uint4 v = {0u, 0u, 0u, 0u};
-	if (i < NB) {
-	  const int part = i & 3, n = (i >> 2) % (16*NT), tp = (i >> 2)/(16*NT);
-	  if (8*part < kc)
-	    v = *reinterpret_cast<const uint4 *>(w + ((int64_t) (3*st + tp)*cout + n0 + n)*cin + c0 + 8*part);
-	}
-	pre[k] = v;
-      }
-    };
-    fetch(0);
-    for (int st = 0; st < 9; st++) {
-#pragma unroll
-      for (int k = 0; k < NBT; k++) {
-	const int i = threadIdx.x + 256*k;
-	if (i < NB) (&sb[0][0][0])[4*(i >> 2) + lds_part(i >> 2, i & 3, swz)] = pre[k];
-      }
-      __syncthreads();                        // halo (first stage) and weights in place
-      if (st + 1 < 9) fetch(st + 1);
-      const int dx = st/3, dy = st%3;
-#pragma unroll
-      for (int dz = 0; dz < 3; dz++) {
-	s8 bv[NT];
-#pragma unroll
-	for (int n = 0; n < NT; n++) {
-	  const int row = dz*16*NT + 16*n + r;
-	  bv[n] = *reinterpret_cast<const s8 *>(&sb[dz][16*n + r][lds_part(row, q, swz)]);
-	}
-#pragma unroll
-	for (int j = 0; j < 4; j++) {
-	  const int h = ((wave + dx)*LH_Y + (j + dy))*LH_Z + (r + dz);
-	  const s8 a = *reinterpret_cast<const s8 *>(&sa[h*4 + lds_part(h, q, swz)]);
-#pragma unroll
-	  for (int n = 0; n < NT; n++)
-	    acc[j][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8, a),
-								 __builtin_bit_cast(b8, bv[n]), acc[j][n], 0, 0, 0);
-	}
-      }
-      __syncthreads();                        // everyone done with this stage's weights
-    }
-  }
-  const int gx = x0 + wave;
-#pragma unroll
-  for (int j = 0; j < 4; j++) {
-    const int gy = y0 + j;
-#pragma unroll
-    for (int n = 0; n < NT; n++) {
-      const int ch = n0 + 16*n + r;
-      const float bv = bias ? bias[ch] : 0.0f;
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-	const int gz = z0 + 4*q + i;
-	if (gx < nx && gy < ny && gz < nz) {
-	  const int64_t p = (((int64_t) b*nx + gx)*ny + gy)*nz + gz;
-	  store_out(y, act, p*cout + ch, acc[j][n][i] + bv, accumulate);
-	}
-      }
-    }
-  }
-}
+typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u4a __attribute__((ext_vector_type(4), aligned(8)));   // 16 bytes, 8-byte aligned
+typedef float f4a __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint16_t h4a __attribute__((ext_vector_type(4), aligned(2)));
 
 // ---------------------------------------------------------------------------
-// Pipelined variant of the LDS-tiled forward pass (the default up to 64
-// output channels per block).  The tiling and the MFMA fragments are those of
-// conv3_fwd_lds_kernel; what changes is where the memory latency goes.
-// rocprof counters of the tiled kernel (MFMA busy 25 % of cycles, waves
-// waiting half their cycles, LDS active a quarter of the time, no bank
-// conflicts) show the halo fill of each input-channel chunk as the binding
-// cost: every block stops for it with nothing to compute.  Here
-//   - the halo of the NEXT input-channel chunk is loaded into registers
-//     while the current chunk is computed, and written to LDS when the
-//     current chunk is done;
-//   - the weights run one stage ahead across chunk boundaries;
-//   - a chunk of 16 channels (cin = 16 mod 32) runs on the K = 16 MFMA
-//     (v_mfma_f32_16x16x16_bf16) instead of a K = 32 one half of zeros.
-// The products and the FP32 accumulation bound are those of the tiled
-// kernel; a 16-channel chunk's MFMA sums 16 products where the tiled
-// kernel's sums them with 16 zero ones, so the last bits may differ.
+// Forward pass (and, on the flipped weights, the backward-data pass).
+//
+// A block works through CT_X x TY x ZT tiles (CT_X = 4*16/ZT) for 16*NT output
+// channels.  Wave w owns TY rows of 16 positions: z0 .. z0+15 at x0 + w
+// (ZT = 16), or 8 z at two neighbouring x (ZT = 8, for lattices up to 8 deep).
+// Input channels go 16 at a time; such a slice of the tile with its halo lies
+// in LDS, 32 bytes per position.
+//
+// A unit is up to two (dx, dz) columns of the stencil, whose 16 channels each
+// fill the K = 32 of v_mfma_f32_16x16x32_bf16: lanes q = 0, 1 hold the first
+// column, q = 2, 3 the second.  Five units make a slice: dz = 0 and 1 for each
+// dx, dz = 2 for dx = 0 and 1, and the ninth column alone (K = 16, which
+// occupies the unit as long: 10 MFMAs do the work of 9).  A unit's weights, three
+// dy taps, are held in registers while the wave walks the TY + 2 halo rows,
+// so one LDS read of a row serves up to 3 taps x NT MFMAs (a read per tap
+// makes LDS the bound: 6 reads per 8 MFMAs at NT = 2).
+//
+// Everything is staged by loads straight to LDS, two buffers each, so no
+// registers hold data in flight: the next unit's weights are requested at a
+// unit's start and waited for at its end; the next slice's halo (of the next
+// tile after the last slice) is requested over the first units of a slice and
+// waited for at its end, the other waits let that unit's halo loads go on.
+//
+// The weights are the first MFMA operand and the positions the second, so
+// lane (r, q) ends with channels 4q .. 4q+3 of position r: 16-byte stores.
+//
+// Bound by the halo loads beside the MFMAs (which are busy 42 % of the time):
+// without them 80 -> 32 channels on 8 x 64^3 would take 264 us.  It takes 357 us
+// (813 TFLOP/s) and the network's 12 layers on 8 x 64^3 0.95 ms, against 500 us
+// and 1.63 ms for a tile per block, staged through registers with two
+// barriers per three taps and a read per tap.
 
-constexpr int HPT = (LH_N*4 + 255)/256;       // halo uint4 per thread
+constexpr int NUNIT = 5;
+constexpr int NXCD = 8;
 
-// One stage (taps dx, dy, dz = 0..2) of the pipelined kernel on the LDS
-// tiles: K = 32 MFMAs on 8-channel fragments.  For a 16-channel chunk taps
-// dz = 0 and 1 share one K = 32 MFMA and tap dz = 2 takes a K = 16 MFMA,
-// lane (r, q) holding channels 4q .. 4q+3 (the (q & 1) half of 16-byte
-// part q >> 1): on gfx950 a K = 16 MFMA occupies the unit as long as a
-// K = 32 one, so the pair saves a third of the chunk's MFMA time.
-template <int NT, bool K16>
-__device__ __forceinline__ void conv_stage(const uint4 * sa, const uint4 (*sb)[16*NT][LK/8], f4 (&acc)[4][NT],
-					   int wave, int r, int q, int dx, int dy, int swz) {
-#pragma unroll
-  for (int dz = 0; dz < 3; dz++) {
-    if constexpr (!K16) {
-      s8 bv[NT];
-#pragma unroll
-      for (int n = 0; n < NT; n++) {
-	const int row = dz*16*NT + 16*n + r;
-	bv[n] = *reinterpret_cast<const s8 *>(&sb[dz][16*n + r][lds_part(row, q, swz)]);
-      }
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-	const int h = ((wave + dx)*LH_Y + (j + dy))*LH_Z + (r + dz);
-	const s8 a = *reinterpret_cast<const s8 *>(&sa[h*4 + lds_part(h, q, swz)]);
-#pragma unroll
-	for (int n = 0; n < NT; n++)
-	  acc[j][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8, a),
-							       __builtin_bit_cast(b8, bv[n]), acc[j][n], 0, 0, 0);
-      }
-    }
-    else if (dz == 0) {
-      // taps dz = 0 and 1 in one K = 32 MFMA: lanes q = 0, 1 hold tap 0's
-      // 16 channels, lanes q = 2, 3 tap 1's (8 channels each, part q & 1)
-      const int dq = q >> 1;
-      s8 bv[NT];
-#pragma unroll
-      for (int n = 0; n < NT; n++) {
-	const int row = dq*16*NT + 16*n + r;
-	bv[n] = *reinterpret_cast<const s8 *>(&sb[dq][16*n + r][lds_part(row, q & 1, swz)]);
-      }
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-	const int h = ((wave + dx)*LH_Y + (j + dy))*LH_Z + (r + dq);
-	const s8 a = *reinterpret_cast<const s8 *>(&sa[h*4 + lds_part(h, q & 1, swz)]);
-#pragma unroll
-	for (int n = 0; n < NT; n++)
-	  acc[j][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8, a),
-							       __builtin_bit_cast(b8, bv[n]), acc[j][n], 0, 0, 0);
-      }
-    }
-    else if (dz == 2) {
-      s4 bv[NT];
-#pragma unroll
-      for (int n = 0; n < NT; n++) {
-	const int row = dz*16*NT + 16*n + r;
-	bv[n] = *reinterpret_cast<const s4 *>(reinterpret_cast<const char *>(&sb[dz][16*n + r][lds_part(row, q >> 1, swz)])
-					      + 8*(q & 1));
-      }
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-	const int h = ((wave + dx)*LH_Y + (j + dy))*LH_Z + (r + dz);
-	const s4 a = *reinterpret_cast<const s4 *>(reinterpret_cast<const char *>(&sa[h*4 + lds_part(h, q >> 1, swz)])
-						   + 8*(q & 1));
-#pragma unroll
-	for (int n = 0; n < NT; n++)
-	  acc[j][n] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, bv[n], acc[j][n], 0, 0, 0);
-      }
-    }
-  }
+template <int TY, int ZT>
+struct ConvTile {
+  static constexpr int XW = 16/ZT;            // x planes of a wave
+  static constexpr int X = 4*XW, HX = X + 2, HY = TY + 2, HZ = ZT + 2;
+  static constexpr int HP = HY*HZ, N = HX*HP; // halo positions of a plane, of the tile
+  static constexpr int HL = (2*N + 63)/64;    // loads of a wave (64 vectors of 16 bytes) in all
+  static constexpr int HW = (HL + 3)/4;       // per wave
+  static constexpr int HU = (HW + NUNIT - 2)/(NUNIT - 1);   // per unit, none in a slice's last
+  static constexpr int in_unit(int u) { return (HW > (u + 1)*HU) ? HU : (HW > u*HU ? HW - u*HU : 0); }
+};
+
+// Weight rows are 4 x 16 bytes, halo rows 2 x 16.  The 16 lanes of a fragment
+// read consecutive rows at one 16-byte part; XOR-swizzling the part with bits
+// of the consecutive index (output channel, z) spreads them over all banks and
+// leaves the other indices plain offsets.
+__device__ __forceinline__ int w_part(int i, int part) { return part ^ ((i >> 1) & 3); }
+__device__ __forceinline__ int h_part(int z, int part) { return part ^ ((z >> 3) & 1); }
+
+// the lattice coordinate of halo offset i: periodic wrap; what lies further
+// out belongs to positions outside the lattice, whose results are dropped
+__device__ __forceinline__ int halo_at(int i, int n) {
+  i = wrapi(i, n);
+  return (i < n) ? i : 0;
 }
 
-// With 16 or 32 output channels per block the kernel is held to 168
-// registers, i.e. 3 blocks (12 waves) per CU as the LDS allows; 48 and 64
-// channels do not fit 168 without spilling and run at 2 blocks per CU;
-// wider blocks take conv3_fwd_lds_kernel.
-template <int NT>
-__global__ void __launch_bounds__(256, (NT <= 2 ? 3 : 2))
-conv3_fwd_pipe_kernel(const uint16_t * __restrict__ x, const uint16_t * __restrict__ w,
-		      const float * __restrict__ bias, float * __restrict__ y, uint16_t * __restrict__ act,
-		      int nx, int ny, int nz, int cin, int cout, int accumulate,
-		      int ntx, int nty, int ntz, int swz) {
-  __shared__ uint4 sa[LH_N*(LK/8)];
-  __shared__ uint4 sb[3][16*NT][LK/8];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int r = lane & 15, q = lane >> 4;
-  int t = blockIdx.x;
-  const int tz = t % ntz; t /= ntz;
-  const int ty = t % nty; t /= nty;
-  const int tx = t % ntx;
-  const int b = t / ntx;
-  const int x0 = tx*LT_X, y0 = ty*LT_Y, z0 = tz*LT_Z;
+// 16 bytes per lane from global memory to LDS at byte offset `to` + 16 lane.
+// The compiler does not know that the load is in flight: wait_barrier waits.
+__device__ __forceinline__ void load_to_lds(const void * from, uint32_t to) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" :: "v"(from), "s"(to) : "memory");
+}
+
+// all but this wave's last N memory operations and all its LDS reads done,
+// then the block barrier
+template <int N>
+__device__ __forceinline__ void wait_barrier() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(N) : "memory");
+}
+
+template <int NT, int TY, int ZT>
+__global__ void __launch_bounds__(256, 2)
+conv3_fwd_kernel(const uint16_t * __restrict__ x, const uint16_t * __restrict__ w,
+		 const float * __restrict__ bias, float * __restrict__ y, uint16_t * __restrict__ act,
+		 int nx, int ny, int nz, int cin, int cout, int accumulate, int ntx, int nty, int ntz, int ntile) {
+  using C = ConvTile<TY, ZT>;
+  constexpr int NW = 3*16*NT*4;               // weight vectors of a unit
+  constexpr int WL = NW/64, WW = (WL + 3)/4;  // loads of a wave: in all, per wave
+  __shared__ u4 lds[2*NW + 2*64*C::HL];       // weights, then halo slices
+  const uint32_t base = (uint32_t) (uintptr_t) (__attribute__((address_space(3))) char *) &lds[0];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 15, q = lane >> 4, hi = q >> 1;
+  const int64_t nsite = (int64_t) nx*ny*nz;
   const int n0 = blockIdx.y*16*NT;
-  constexpr int NB = 3*16*NT*(LK/8);
-  constexpr int NBT = (NB + 255)/256;
-  const uint16_t * xb = x + (int64_t) b*nx*ny*nz*cin;
 
-  // halo of chunk c0 into registers
-  uint4 hpre[HPT];
-  auto fetch_halo = [&](int c0) {
-    const int kc = (cin - c0 < LK) ? cin - c0 : LK;
+  // This lane's halo vectors: load i of the wave covers vectors 64 j .. + 63,
+  // j = wave + 4 i, two per position.  Loads and positions past the end repeat
+  // the last ones, so that every wave issues as many.
+  int hc[C::HW];                              // halo coordinates and part
+  uint32_t hs[C::HW];                         // site in the tile being fetched
 #pragma unroll
-    for (int k = 0; k < HPT; k++) {
-      const int i = threadIdx.x + 256*k;
-      const int h = i >> 2, part = i & 3;
-      uint4 v = {0u, 0u, 0u, 0u};
-      if (i < LH_N*4 && 8*part < kc) {
-	const int hz = h % LH_Z, hy = (h / LH_Z) % LH_Y, hx = h / (LH_Z*LH_Y);
-	const int gx = wrapi(x0 + hx - 1, nx), gy = wrapi(y0 + hy - 1, ny), gz = wrapi(z0 + hz - 1, nz);
-	v = *reinterpret_cast<const uint4 *>(xb + (((int64_t) gx*ny + gy)*nz + gz)*cin + c0 + 8*part);
-      }
-      hpre[k] = v;
+  for (int i = 0; i < C::HW; i++) {
+    const int v = 64*min(wave + 4*i, C::HL - 1) + lane;
+    const int p = min(v >> 1, C::N - 1);
+    const int hz = p % C::HZ, hy = (p/C::HZ) % C::HY, hx = p/C::HP;
+    hc[i] = hx | (hy << 8) | (hz << 16) | (h_part(hz, v & 1) << 24);
+  }
+  int x0, y0, z0;
+  int64_t p0;                                 // first position of the sample
+  auto locate = [&](int t, int & tx, int & ty, int & tz, int64_t & tp) {
+    tz = (t % ntz)*ZT; t /= ntz;
+    ty = (t % nty)*TY; t /= nty;
+    tx = (t % ntx)*C::X;
+    tp = (int64_t) (t/ntx)*nsite;
+  };
+  auto sites = [&](int tx, int ty, int tz) {
+#pragma unroll
+    for (int i = 0; i < C::HW; i++) {
+      const int cx = halo_at(tx + (hc[i] & 255) - 1, nx), cy = halo_at(ty + ((hc[i] >> 8) & 255) - 1, ny);
+      hs[i] = ((uint32_t) cx*ny + cy)*nz + halo_at(tz + ((hc[i] >> 16) & 255) - 1, nz);
     }
   };
-  auto store_halo = [&]() {
+  // loads [i0, i1) of slice c0 of the sample at tp into halo buffer hb
+  auto fetch_halo = [&](int i0, int i1, int64_t tp, int c0, int hb) {
 #pragma unroll
-    for (int k = 0; k < HPT; k++) {
-      const int i = threadIdx.x + 256*k;
-      if (i < LH_N*4) sa[4*(i >> 2) + lds_part(i >> 2, i & 3, swz)] = hpre[k];
-    }
-  };
-  // weights of taps 3st .. 3st+2 of chunk c0: [tap][n][part]
-  uint4 wpre[NBT];
-  auto fetch_w = [&](int c0, int st) {
-    const int kc = (cin - c0 < LK) ? cin - c0 : LK;
-#pragma unroll
-    for (int k = 0; k < NBT; k++) {
-      const int i = threadIdx.x + 256*k;
-      uint4 v = {0u, 0u, 0u, 0u};
-      if (i < NB) {
-	const int part = i & 3, n = (i >> 2) % (16*NT), tp = (i >> 2)/(16*NT);
-	if (8*part < kc)
-	  v = *reinterpret_cast<const uint4 *>(w + ((int64_t) (3*st + tp)*cout + n0 + n)*cin + c0 + 8*part);
-      }
-      wpre[k] = v;
-    }
-  };
-  auto store_w = [&]() {
-#pragma unroll
-    for (int k = 0; k < NBT; k++) {
-      const int i = threadIdx.x + 256*k;
-      if (i < NB) (&sb[0][0][0])[4*(i >> 2) + lds_part(i >> 2, i & 3, swz)] = wpre[k];
+    for (int i = 0; i < C::HW; i++) {
+      if (i < i0 || i >= i1) continue;
+      load_to_lds(x + (tp + hs[i])*cin + (c0 + 8*(hc[i] >> 24)),
+		  base + 16*(2*NW + 64*(hb*C::HL + min(wave + 4*i, C::HL - 1))));
     }
   };
 
-  f4 acc[4][NT];
+  // This lane's weight vectors: row dy*16*NT + n, part; parts 2, 3 belong to
+  // the unit's second column.  Rows past the last output channel repeat it.
+  int wo[WW];
+  const int tap = cout*cin;
 #pragma unroll
-  for (int j = 0; j < 4; j++)
+  for (int k = 0; k < WW; k++) {
+    const int i = 64*min(wave + 4*k, WL - 1) + lane;
+    const int row = i >> 2, part = w_part(row, i & 3);
+    const int n = min(n0 + row % (16*NT), cout - 1);
+    wo[k] = ((3*(row/(16*NT))*cout + n)*cin + 8*(part & 1))*2 + (part >> 1);
+  }
+  auto fetch_w = [&](int u, int c0, int buf) {
+    // second column: dz + 1 (units 0-2), dx + 1 (unit 3), none (unit 4)
+    const int col = (u < 3) ? 9*u : (u == 3 ? 2 : 20), step = (u < 3) ? 1 : (u == 3 ? 9 : 0);
+#pragma unroll
+    for (int k = 0; k < WW; k++)
+      load_to_lds(w + ((int64_t) col*tap + c0) + ((wo[k] >> 1) + (wo[k] & 1)*(step*tap)),
+		  base + 16*(buf*NW + 64*min(wave + 4*k, WL - 1)));
+  };
+
+  f4 acc[TY][NT];
+#pragma unroll
+  for (int j = 0; j < TY; j++)
 #pragma unroll
     for (int n = 0; n < NT; n++) acc[j][n] = f4{0.0f, 0.0f, 0.0f, 0.0f};
 
-  // full 32-channel chunks; the halo of the next chunk (full or not) is
-  // loaded while this one is computed, the weights one stage ahead
-  const int cfull = cin - cin % LK;
-  fetch_halo(0);
-  fetch_w(0, 0);
-#pragma unroll 1
-  for (int c0 = 0; c0 < cfull; c0 += LK) {
-    // every wave is done with the previous chunk's halo (barrier at the
-    // end of its last stage)
-    store_halo();
-    if (c0 + LK < cin) fetch_halo(c0 + LK);
-#pragma unroll 1
-    for (int st = 0; st < 9; st++) {
-      store_w();
-      __syncthreads();                        // halo (first stage) and weights in place
-      if (st + 1 < 9) fetch_w(c0, st + 1);
-      else if (c0 + LK < cin) fetch_w(c0 + LK, 0);
-      conv_stage<NT, false>(sa, sb, acc, wave, r, q, st/3, st%3, swz);
-      __syncthreads();                        // everyone done with this stage's weights
-    }
-  }
-  // a last chunk of 16 channels
-  if (cfull < cin) {
-    store_halo();
-#pragma unroll 1
-    for (int st = 0; st < 9; st++) {
-      store_w();
-      __syncthreads();
-      if (st + 1 < 9) fetch_w(cfull, st + 1);
-      conv_stage<NT, true>(sa, sb, acc, wave, r, q, st/3, st%3, swz);
-      __syncthreads();
-    }
-  }
-  const int gx = x0 + wave;
+  // halo row of lane r in this wave's row Y = 0, column (dx, dz) = (0, 0)
+  const int rz = (ZT == 16) ? r : (r & 7), rx = C::XW*wave + (ZT == 16 ? 0 : r >> 3);
+  const int hrow = rx*C::HP + rz;
+  auto unit32 = [&](int buf, int hb, int dx, int dz) {
+    const u4 * pw = &lds[buf*NW + 4*r + w_part(r, q)];
+    const u4 * pa = &lds[2*NW + 64*C::HL*hb + 2*(hrow + dx*C::HP + dz) + h_part(rz + dz, q & 1)];
+    b8 bw[3][NT];
 #pragma unroll
-  for (int j = 0; j < 4; j++) {
-    const int gy = y0 + j;
+    for (int dy = 0; dy < 3; dy++)
+#pragma unroll
+      for (int n = 0; n < NT; n++) bw[dy][n] = __builtin_bit_cast(b8, pw[64*(dy*NT + n)]);
+#pragma unroll
+    for (int Y = 0; Y < TY + 2; Y++) {
+      const b8 a = __builtin_bit_cast(b8, pa[2*Y*C::HZ]);
+#pragma unroll
+      for (int dy = 0; dy < 3; dy++) {
+	const int j = Y - dy;
+	if (j < 0 || j >= TY) continue;
+#pragma unroll
+	for (int n = 0; n < NT; n++)
+	  acc[j][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bw[dy][n], a, acc[j][n], 0, 0, 0);
+      }
+    }
+  };
+  // the ninth column: lane (r, q) holds channels 4q .. 4q+3, the (q & 1) half
+  // of part q >> 1
+  auto unit16 = [&](int buf, int hb) {
+    auto half = [&](const u4 * v) {
+      return *reinterpret_cast<const s4 *>(reinterpret_cast<const char *>(v) + 8*(q & 1));
+    };
+    const u4 * pw = &lds[buf*NW + 4*r + w_part(r, hi)];
+    const u4 * pa = &lds[2*NW + 64*C::HL*hb + 2*(hrow + 2*C::HP + 2) + h_part(rz + 2, hi)];
+    s4 bw[3][NT];
+#pragma unroll
+    for (int dy = 0; dy < 3; dy++)
+#pragma unroll
+      for (int n = 0; n < NT; n++) bw[dy][n] = half(pw + 64*(dy*NT + n));
+#pragma unroll
+    for (int Y = 0; Y < TY + 2; Y++) {
+      const s4 a = half(pa + 2*Y*C::HZ);
+#pragma unroll
+      for (int dy = 0; dy < 3; dy++) {
+	const int j = Y - dy;
+	if (j < 0 || j >= TY) continue;
+#pragma unroll
+	for (int n = 0; n < NT; n++)
+	  acc[j][n] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(bw[dy][n], a, acc[j][n], 0, 0, 0);
+      }
+    }
+  };
+
+  // results of the tile: lane (r, q) has channels 4q .. 4q+3 of position r of
+  // each row
+  auto store_tile = [&]() {
+    const int gx = x0 + rx, gz = z0 + rz;
+    if (gx >= nx || gz >= nz) return;
+    const int64_t o0 = (p0 + ((int64_t) gx*ny + y0)*nz + gz)*cout + n0 + 4*q;
 #pragma unroll
     for (int n = 0; n < NT; n++) {
-      const int ch = n0 + 16*n + r;
-      const float bv = bias ? bias[ch] : 0.0f;
+      if (n0 + 16*n >= cout) continue;
+      f4 bv = f4{0.0f, 0.0f, 0.0f, 0.0f};
+      if (bias) bv = *reinterpret_cast<const f4a *>(bias + n0 + 16*n + 4*q);
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-	const int gz = z0 + 4*q + i;
-	if (gx < nx && gy < ny && gz < nz) {
-	  const int64_t p = (((int64_t) b*nx + gx)*ny + gy)*nz + gz;
-	  store_out(y, act, p*cout + ch, acc[j][n][i] + bv, accumulate);
+      for (int j = 0; j < TY; j++) {
+	if (y0 + j >= ny) continue;
+	const int64_t o = o0 + (int64_t) j*nz*cout + 16*n;
+	f4 v = acc[j][n] + bv;
+	if (y) {
+	  f4a * yo = reinterpret_cast<f4a *>(y + o);
+	  if (accumulate) v += f4(*yo);
+	  *yo = v;
+	}
+	if (act) {
+	  h4a a;
+#pragma unroll
+	  for (int i = 0; i < 4; i++) a[i] = silu_bf16(v[i]);
+	  *reinterpret_cast<h4a *>(act + o) = a;
 	}
       }
     }
+  };
+
+  // Blocks are dispatched round-robin over the 8 XCDs.  Where the grid allows,
+  // XCD g takes the tiles [g per, (g + 1) per) in order, all its blocks side by
+  // side, so that neighbouring tiles share their halos and the 128-byte lines
+  // of their slices in its L2.
+  const bool xcd = (gridDim.x % NXCD == 0);
+  const int per = xcd ? (ntile + NXCD - 1)/NXCD : ntile;
+  const int step = xcd ? (int) gridDim.x/NXCD : (int) gridDim.x;
+  const int first = xcd ? (int) (blockIdx.x % NXCD)*per : 0;
+  const int end = min(first + per, ntile);
+  int tile = first + (xcd ? (int) blockIdx.x/NXCD : (int) blockIdx.x);
+  if (tile >= end) return;
+  locate(tile, x0, y0, z0, p0);
+  sites(x0, y0, z0);
+  fetch_w(0, 0, 0);
+  fetch_halo(0, C::HW, p0, 0, 0);
+  wait_barrier<0>();
+  int buf = 0, hb = 0, c0 = 0;
+#pragma unroll 1
+  for (;;) {
+    // the slice that follows; after the block's last one, that one again (not
+    // used, but every unit then waits for the same number of loads)
+    const bool last = (c0 + 16 >= cin);
+    const bool done = last && (tile + step >= end);
+    const int cn = done ? c0 : (last ? 0 : c0 + 16);
+    const int tn = (last && !done) ? tile + step : tile;
+    int xn = x0, yn = y0, zn = z0;
+    int64_t pn = p0;
+    if (last) {
+      locate(tn, xn, yn, zn, pn);
+      sites(xn, yn, zn);
+    }
+#pragma unroll
+    for (int u = 0; u < NUNIT; u++) {
+      if (u + 1 < NUNIT) fetch_w(u + 1, c0, buf ^ 1);
+      else fetch_w(0, cn, buf ^ 1);
+      if (u + 1 < NUNIT) fetch_halo(u*C::HU, (u + 1)*C::HU, pn, cn, hb ^ 1);
+      if (u < 3) unit32(buf, hb, u, hi);
+      else if (u == 3) unit32(buf, hb, hi, 2);
+      else unit16(buf, hb);
+      // wait for the weights; this unit's halo loads may go on
+      if (u == 0) wait_barrier<C::in_unit(0)>();
+      else if (u == 1) wait_barrier<C::in_unit(1)>();
+      else if (u == 2) wait_barrier<C::in_unit(2)>();
+      else if (u == 3) wait_barrier<C::in_unit(3)>();
+      else wait_barrier<0>();
+      buf ^= 1;
+    }
+    if (last) {
+      store_tile();
+      if (done) break;
+#pragma unroll
+      for (int j = 0; j < TY; j++)
+#pragma unroll
+	for (int n = 0; n < NT; n++) acc[j][n] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    hb ^= 1;
+    tile = tn;
+    c0 = cn;
+    x0 = xn; y0 = yn; z0 = zn; p0 = pn;
   }
 }
 
@@ -510,9 +368,6 @@ conv3_fwd_pipe_kernel(const uint16_t * __restrict__ x, const uint16_t * __restri
 // 133 us (1.09 PFLOP/s), and the 12 layers of the network 0.52 ms with the
 // reductions, against 14.6 ms when every block staged its positions again
 // for each tap and transposed the fragments with 2-byte LDS reads.
-
-typedef uint32_t u4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u4a __attribute__((ext_vector_type(4), aligned(8)));   // 16 bytes, 8-byte aligned
 
 constexpr int WT_Y = 8, WT_Z = 16;
 constexpr int WT_N = WT_Y*WT_Z;                       // positions of a tile plane
@@ -741,31 +596,55 @@ __global__ void to_bf16_kernel(const float * __restrict__ a, uint16_t * __restri
     b[i] = to_bf16(a[i]);
 }
 
-// LDS swizzle shift of the tiled kernel (LDW_CONV_SWZ; 16 = no swizzle)
-int conv_swz() {
-  static int v = -1;
-  if (v < 0) {
-    const char * e = getenv("LDW_CONV_SWZ");
-    v = e ? atoi(e) : 1;
-  }
-  return v;
-}
-
-// LDW_CONV_LDS=0 selects the fragment-direct kernel everywhere, =1 the
-// tiled kernel without the pipeline (A/B timing); by default the
-// pipelined kernel (up to 64 output channels per block)
-int conv_lds_enabled() {
-  static int on = -1;
-  if (on < 0) {
-    const char * e = getenv("LDW_CONV_LDS");
-    on = e ? atoi(e) : 2;
-  }
-  return on;
-}
-
 int grid_for(int64_t n) {
   int64_t g = (n + 255)/256;
   return (int) (g < 8192 ? (g > 0 ? g : 1) : 8192);
+}
+
+constexpr int CONV_BLOCKS = 512;              // two per CU
+
+struct ConvShape { int nt, ty, zt; };
+
+// Output channels per block (16 nt), rows per wave and depth of the tile.
+//
+// A wave wants 8 rows (a halo row is then read 1.25 times instead of 1.5) as
+// long as that makes enough blocks, with up to 32 channels: 8 rows and 48 do
+// not fit LDS twice.  80 -> 32 channels on 8 x 64^3: 357 us with (2, 8), 396
+// with (2, 4), 459 with (1, 8).  Wider layers take 3 or 4 blocks of 16,
+// whichever pads less (32 -> 48 on 8 x 32^3: 32 us with nt = 3, 37 with 2, 36
+// with 4), and fewer where the grid would not give each CU two blocks (64 ->
+// 64 on 8 x 16^3: 22 us with nt = 4, 17 with 2 or 1).
+ConvShape conv_shape(int batch, int nx, int ny, int nz, int nb16) {
+  ConvShape c;
+  c.zt = (nz > 8) ? 16 : 8;
+  const int cx = 4*16/c.zt;
+  auto tiles = [&](int ty) {
+    return (int64_t) batch*((nx + cx - 1)/cx)*((ny + ty - 1)/ty)*((nz + c.zt - 1)/c.zt);
+  };
+  c.ty = 4;
+  if (nb16 <= 2) {
+    c.nt = nb16;
+    if (tiles(8) >= CONV_BLOCKS) c.ty = 8;
+  }
+  else {
+    c.nt = ((nb16 + 3)/4*4 <= (nb16 + 2)/3*3) ? 4 : 3;
+  }
+  while (c.nt > 1 && tiles(c.ty)*((nb16 + c.nt - 1)/c.nt) < CONV_BLOCKS) c.nt--;
+  return c;
+}
+
+template <int NT, int TY, int ZT>
+void launch_conv(const uint16_t * x, const uint16_t * w, const float * bias, float * y, uint16_t * act,
+		 int batch, int nx, int ny, int nz, int cin, int cout, int accumulate, hipStream_t s) {
+  constexpr int X = ConvTile<TY, ZT>::X;
+  const int ntx = (nx + X - 1)/X, nty = (ny + TY - 1)/TY, ntz = (nz + ZT - 1)/ZT;
+  const int ntile = batch*ntx*nty*ntz, nb = (cout/16 + NT - 1)/NT;
+  int nblk = CONV_BLOCKS/nb;
+  if (nblk < 1) nblk = 1;
+  if (nblk >= NXCD) nblk -= nblk % NXCD;
+  if (nblk > ntile) nblk = ntile;
+  hipLaunchKernelGGL((conv3_fwd_kernel<NT, TY, ZT>), dim3(nblk, nb), dim3(256), 0, s, x, w, bias, y, act, nx, ny, nz,
+		     cin, cout, accumulate, ntx, nty, ntz, ntile);
 }
 
 }  // namespace
@@ -773,58 +652,24 @@ int grid_for(int64_t n) {
 hipError_t launch_conv3_fwd(const uint16_t * x, const uint16_t * w, const float * bias, float * y,
 			    uint16_t * act, int batch, int nx, int ny, int nz, int cin, int cout,
 			    int accumulate, hipStream_t s) {
-  const int64_t npos = (int64_t) batch*nx*ny*nz;
   const int nb16 = cout/16;
-  if (nz >= LT_Z && ny >= LT_Y && nx >= LT_X && conv_lds_enabled()) {
-    int nt = 1;
-    for (int c = LNT_MAX; c >= 1; c--) if (nb16 % c == 0) { nt = c; break; }
-    const int ntx = (nx + LT_X - 1)/LT_X, nty = (ny + LT_Y - 1)/LT_Y, ntz = (nz + LT_Z - 1)/LT_Z;
-    dim3 grid((unsigned) ((int64_t) batch*ntx*nty*ntz), nb16/nt), block(256);
-    if (conv_lds_enabled() == 2 && nt <= 4) {
-#define PIPE_(NT) hipLaunchKernelGGL(conv3_fwd_pipe_kernel<NT>, grid, block, 0, s, x, w, bias, y, act, nx, ny, nz, \
-				     cin, cout, accumulate, ntx, nty, ntz, conv_swz())
-      switch (nt) {
-      case 4: PIPE_(4); break;
-      case 3: PIPE_(3); break;
-      case 2: PIPE_(2); break;
-      default: PIPE_(1); break;
-      }
-#undef PIPE_
-      return hipGetLastError();
+  const ConvShape c = conv_shape(batch, nx, ny, nz, nb16);
+#define CONV_(NT, TY, ZT) launch_conv<NT, TY, ZT>(x, w, bias, y, act, batch, nx, ny, nz, cin, cout, accumulate, s)
+#define CONV_NT(NT, TY) do { if (c.zt == 16) CONV_(NT, TY, 16); else CONV_(NT, TY, 8); } while (0)
+  if (c.ty == 8) {
+    if (c.nt == 2) CONV_NT(2, 8);
+    else CONV_NT(1, 8);
+  }
+  else {
+    switch (c.nt) {
+    case 4: CONV_NT(4, 4); break;
+    case 3: CONV_NT(3, 4); break;
+    case 2: CONV_NT(2, 4); break;
+    default: CONV_NT(1, 4); break;
     }
-#define LDS_(NT) hipLaunchKernelGGL(conv3_fwd_lds_kernel<NT>, grid, block, 0, s, x, w, bias, y, act, nx, ny, nz, \
-				    cin, cout, accumulate, ntx, nty, ntz, conv_swz())
-    switch (nt) {
-    case 6: LDS_(6); break;
-    case 5: LDS_(5); break;
-    case 4: LDS_(4); break;
-    case 3: LDS_(3); break;
-    case 2: LDS_(2); break;
-    default: LDS_(1); break;
-    }
-#undef LDS_
-    return hipGetLastError();
   }
-  // small lattices (the network's coarsest level): fewer output blocks
-  // per wave and fewer waves per block, so that the grid still spreads
-  // over the CUs (at 8 x 8^3 positions, 64 -> 96 channels: 768 one-wave
-  // blocks instead of 64 four-wave ones)
-  int nt = (nb16 % 4 == 0) ? 4 : (nb16 % 3 == 0) ? 3 : (nb16 % 2 == 0) ? 2 : 1;
-  int wpb = 4;
-  const int64_t want = 1024;
-  while (wpb > 1 && ((npos + 32*wpb - 1)/(32*wpb))*(nb16/nt) < want) wpb /= 2;
-  while (nt > 1 && ((npos + 32*wpb - 1)/(32*wpb))*(nb16/nt) < want) {
-    int c = nt - 1;
-    while (c > 1 && nb16 % c) c--;
-    nt = c;
-  }
-  dim3 grid((unsigned) ((npos + 32*wpb - 1)/(32*wpb)), nb16/nt), block(64*wpb);
-  switch (nt) {
-  case 4: hipLaunchKernelGGL(conv3_fwd_kernel<4>, grid, block, 0, s, x, w, bias, y, act, npos, nx, ny, nz, cin, cout, accumulate); break;
-  case 3: hipLaunchKernelGGL(conv3_fwd_kernel<3>, grid, block, 0, s, x, w, bias, y, act, npos, nx, ny, nz, cin, cout, accumulate); break;
-  case 2: hipLaunchKernelGGL(conv3_fwd_kernel<2>, grid, block, 0, s, x, w, bias, y, act, npos, nx, ny, nz, cin, cout, accumulate); break;
-  default: hipLaunchKernelGGL(conv3_fwd_kernel<1>, grid, block, 0, s, x, w, bias, y, act, npos, nx, ny, nz, cin, cout, accumulate); break;
-  }
+#undef CONV_NT
+#undef CONV_
   return hipGetLastError();
 }
 

@@ -9,6 +9,7 @@
 #include <stdint.h>
 
 #include "kernels.h"
+#include "silu.h"
 
 namespace ldw {
 
@@ -35,10 +36,7 @@ int grid_of(int64_t n) {
 
 // SiLU: a = z sigma(z)
 __global__ void silu_fwd_kernel(const float * __restrict__ z, uint16_t * __restrict__ a, int64_t n) {
-  GRID_STRIDE(i, n) {
-    const float v = z[i];
-    a[i] = bf16_of(v/(1.0f + expf(-v)));
-  }
+  GRID_STRIDE(i, n) a[i] = silu_bf16(z[i]);
 }
 
 // dz = da sigma(z) (1 + z (1 - sigma(z)))

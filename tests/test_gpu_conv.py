@@ -31,6 +31,11 @@ def vp(d):
     return ctypes.c_void_p(d.ptr)
 
 
+def at(d, nbytes):
+    """The device address nbytes into d."""
+    return ctypes.c_void_p(d.ptr + nbytes)
+
+
 def within(got, want, bound, what):
     err = np.abs(got - want)
     bad = np.flatnonzero(err > bound)
@@ -96,6 +101,35 @@ def test_conv_fwd_bwd_against_oracle(cin, cout, batch, shape):
     within(y.download().astype(np.float64), 2 * yo, 4 * 27 * cin * EPS32 * ya + 1e-30, "forward x2")
 
 
+# the forward tiles: 4 or 8 rows of 16 z or 2 x 8 z per wave, 4 (or 8) x deep;
+# lattices of one site, one below, at and one above a tile's edges, slices
+# that end on 16 channels, output blocks that pad (5, 7), more tiles than
+# blocks (the last shapes: 8-row tiles and 16-channel outputs), in an order of
+# tiles that does and does not divide by the 8 XCDs; off shifts x and w off
+# 16-byte alignment
+@pytest.mark.parametrize("cin,cout,batch,shape,off", [
+    (16, 16, 1, (1, 1, 1), 0), (16, 32, 1, (3, 3, 7), 1), (32, 16, 1, (4, 4, 8), 0), (48, 80, 1, (9, 5, 8), 0),
+    (16, 48, 2, (5, 5, 9), 1), (32, 112, 1, (4, 3, 17), 0), (64, 64, 1, (2, 9, 16), 0), (16, 128, 1, (1, 4, 31), 0),
+    (16, 32, 5, (33, 9, 48), 0), (32, 16, 3, (37, 33, 40), 0), (16, 48, 4, (17, 33, 50), 0)])
+def test_conv_forward_tiles(cin, cout, batch, shape, off):
+    lib = L.lib()
+    rng = np.random.default_rng(3 * cin + cout + shape[2])
+    n = batch * int(np.prod(shape))
+    x, w = bf16_round(rng.standard_normal(n * cin)), bf16_round(rng.standard_normal(27 * cout * cin))
+    bias = rng.standard_normal(cout).astype(np.float32)
+    before = rng.standard_normal(n * cout).astype(np.float32)
+    pad = np.zeros(4 * off, np.uint16)
+    dx, dw = dev(np.concatenate([pad, bf16_bits(x)]), np.uint16), dev(np.concatenate([pad, bf16_bits(w)]), np.uint16)
+    db, dy = dev(bias, np.float32), dev(before, np.float32)
+    print(f"forward cin={cin} cout={cout} batch={batch} shape={shape}", flush=True)
+    want = O.conv3_fwd(x, w, bias.astype(np.float64), shape, cin, cout, batch)
+    mag = O.conv3_fwd(np.abs(x), np.abs(w), np.abs(bias.astype(np.float64)), shape, cin, cout, batch)
+    for acc in (1, 0):
+        assert lib.ldw_conv3d_fwd(at(dx, 8 * off), at(dw, 8 * off), vp(db), vp(dy), batch, *shape, cin, cout, acc) == 0
+        within(dy.download().astype(np.float64), want + acc * before,
+               2 * (27 * cin + 2) * EPS32 * (mag + acc * np.abs(before)) + 1e-30, f"forward accumulate={acc}")
+
+
 # the weight gradient's tiles are 8 x 16 (y, z) columns marched along x: one
 # site, ragged tiles on both sides of an edge, single planes, uneven x ranges,
 # either operand shifted, one to ten 16-channel blocks of the fixed operand
@@ -119,11 +153,6 @@ def test_conv_weight_gradient_tiles(cin, cout, batch, shape, accumulate):
     if accumulate:
         want, mag = want + before, mag + np.abs(before)
     within(dw.download().astype(np.float64), want, 2 * (n + 1) * EPS32 * mag + 1e-30, "weight gradient")
-
-
-def at(d, nbytes):
-    """The device address nbytes into d."""
-    return ctypes.c_void_p(d.ptr + nbytes)
 
 
 # channel counts below, at and above what a block's 256 threads cover, 4 at a
