@@ -4,7 +4,7 @@
 // force from phi_t, the Cahn-Hilliard update phi_t -> phi_t+1 with the
 // velocity of the previous collision, the collision of f_t with that force
 // (giving rho_t, u_t), and the propagation.  Here one block owns a tile of
-// (y, z) columns (8 x 64 by default) and marches along x through a chunk of planes
+// (y, z) columns and marches along x through a chunk of planes
 // (step_tile.h): for each site it forms F and the new phi from the LDS
 // tiles, then collides the site's 19 pulled distributions with that F.  The
 // force never goes to memory.
@@ -29,7 +29,7 @@ using namespace tile;
 
 template <typename T, class S, int ORDER, int METHOD, bool GZ, bool CONS, bool GMU>
 __global__ void __launch_bounds__(S::NT)
-binary_step_kernel(Geom g, FeParams fe, LbParams prm, int xchunk, int nbz, int nby, int nbx, int remap,
+binary_step_kernel(Geom g, FeParams fe, LbParams prm, int nbz, int nby, int nbx, int remap,
 		   const T * __restrict__ phi, T * __restrict__ phi_out,
 		   const T * __restrict__ u_prev, T * __restrict__ u_next,
 		   T * __restrict__ rho, const T * __restrict__ g_in,
@@ -39,8 +39,10 @@ binary_step_kernel(Geom g, FeParams fe, LbParams prm, int xchunk, int nbz, int n
 
   int bzi, byi, bxi;
   if (!tile_of_block(nbz, nby, nbx, remap, bzi, byi, bxi)) return;
-  const int xb = bxi*xchunk;
-  const int xe = min(xb + xchunk, g.nx);
+  // nbx chunks of planes, even to within one plane
+  const int xq = g.nx/nbx, xr = g.nx - xq*nbx;
+  const int xb = bxi*xq + min(bxi, xr);
+  const int xe = xb + xq + (bxi < xr ? 1 : 0);
   step_tile<T, S, ORDER, METHOD, GZ, CONS, GMU>(s, g, fe, prm, byi*S::TY, bzi*S::TZ, xb, xe, phi, phi_out,
 					   u_prev, u_next, rho, g_in, g_out, fz0, fz1, fz2, csum);
 }
@@ -64,46 +66,102 @@ int resident_slots() {
   return slots;
 }
 
-// Planes per block.  A block that marches over xchunk planes first loads
-// 4 phi planes and forms 2 Q planes (about 3 planes of work), so a launch
-// costs about ceil(nblocks/slots)*(xchunk + 3) plane-times: the chunk that
-// minimises it balances the prologue against the last, partly filled round
-// of blocks (on MI355X 3.6 % faster than a fixed 2048-block grid at 256^3
-// FP64, 3.4 % at 128^3 FP32).
-inline int step_xchunk(int nx, int64_t ncol, int slots) {
-  int best = nx;
+inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1)/b; }
+
+// Chunks of x planes for 64 x 8 tiles of a lattice that takes many rounds of
+// blocks.  A block that marches over xc planes first loads 4 phi planes and
+// forms 2 Q planes (about 3 planes of work), so a launch costs about
+// ceil(blocks/slots)*(xc + 3) plane-times; the chunk that minimises it
+// balances the prologue against the last, partly filled round (on MI355X
+// 3.6 % faster than a fixed 2048-block grid at 256^3 FP64, 3.4 % at 128^3
+// FP32).
+//
+// remap: the XCD-contiguous tile order, unless a chunk has more column tiles
+// than an XCD holds blocks and the XCDs would share chunks (192^3 FP64, 7
+// chunks of 72 columns: 534 us in linear order, 545 contiguous; 122x46x214, 10
+// chunks of 24: 138 and 122).
+struct StepPlan { int tz, nchunk, remap; };
+
+inline StepPlan rounds_plan(const Geom & g, int slots) {
+  const int nx = g.nx;
+  const int64_t ncol = ceil_div(g.nz, 64)*ceil_div(g.ny, 8);
+  int best = 1;
   int64_t best_cost = -1;
   for (int xc = nx; ; xc = (xc + 1)/2) {
-    const int64_t nblk = ncol*((nx + xc - 1)/xc);
-    const int64_t cost = ((nblk + slots - 1)/slots)*(int64_t) (xc + 3);
-    if (best_cost < 0 || cost <= best_cost) { best = xc; best_cost = cost; }
-    if (xc <= 4) break;
+    const int n = (int) ceil_div(nx, xc);
+    const int64_t cost = ceil_div(ncol*n, slots)*(xc + 3);
+    if (best_cost < 0 || cost <= best_cost) { best = n; best_cost = cost; }
+    if (xc <= 1) break;
   }
-  return best;
+  return {64, best, (8*ncol <= slots || best % 8 == 0) ? 1 : 0};
+}
+
+// The tile (its z extent; 8 rows in y) and the number of x chunks.
+//
+// A small lattice is bound by the length of one block: prologue and planes in
+// a row.  It takes one round of blocks with as few planes each as fill the
+// resident slots (2 blocks of 32 x 8 or 4 of 16 x 8 threads fit where one of
+// 64 x 8 does), of the tile whose padding in y and z leaves the fewest planes
+// per block.  A large one is bound by memory: 64-wide rows where z pads little,
+// with long chunks; else 32-wide ones with chunks of 3 planes, so that
+// neighbouring tiles of an XCD run close together and share their edge lines
+// in its L2.  Measured over 60 lattices of 16^3 to 256^3, cubic and ragged (us
+// per step, with one 64 x 8 tile of at least 4 planes before): FP64 32^3 28.9 ->
+// 9.7, 64^3 33 -> 22, 80^3 65 -> 42, 91x88x66 92 -> 46, 102x221x150 375 -> 333,
+// 128^3 174 -> 171, 256^3 unchanged; FP32 64^3 22 -> 15, 96^3 52 -> 34,
+// 144^3 223 -> 153.  The best of all tiles and chunks is 3 % (FP64) and 6 %
+// (FP32) faster on average.  The lines between the two: at 0.8 M sites (FP64;
+// 1.0 M: 87x78x169 137 us in one round of 16 x 8 tiles, 109 in 64 x 8 chunks)
+// and 1.25 M (FP32), and at 1.2 of padding (FP64 87x58x212, 1.21: 104 us with 64
+// x 8, 108 with 32 x 8; 82x173x150, 1.28: 237 and 209).
+template <typename T>
+StepPlan step_plan(const Geom & g) {
+  static const int tzs[3] = {16, 32, 64};
+  const int slots[3] = {resident_slots<T, Shape<16, 8>>(), resident_slots<T, Shape<32, 8>>(),
+			resident_slots<T, Shape<64, 8>>()};
+  // a plane of the narrower tiles costs slightly more or less than its share
+  static const double weight64[3] = {1.00, 1.02, 1.10}, weight32[3] = {1.05, 1.00, 1.10};
+  const double * weight = (sizeof(T) == 8) ? weight64 : weight32;
+  const int64_t small = (sizeof(T) == 8) ? 800000 : 1250000;
+  const int forced = tune_step_tile();
+  if (g.nsite <= small || forced) {
+    StepPlan best = {0, 0, 1};
+    double best_cost = 0.0;
+    for (int k = 0; k < 3; k++) {
+      if (forced && tzs[k] != forced) continue;
+      const int64_t ncol = ceil_div(g.nz, tzs[k])*ceil_div(g.ny, 8);
+      if (slots[k] < ncol) continue;
+      const int64_t xc = ceil_div(g.nx, slots[k]/ncol);
+      const double cost = (double) (xc + 2)*weight[k];
+      if (best.tz == 0 || cost < best_cost) { best = {tzs[k], (int) ceil_div(g.nx, xc), 1}; best_cost = cost; }
+    }
+    if (best.tz && g.nsite <= small) return best;
+  }
+  if (forced == 64 || (!forced && ceil_div(g.nz, 64)*64*5 <= (int64_t) g.nz*6))
+    return rounds_plan(g, slots[2]);
+  return {forced ? forced : 32, (int) ceil_div(g.nx, 3), 1};
 }
 
 template <typename T, class S, bool CONS, bool GMU = false>
 void launch_shape(const Geom & g, const FeParams & fe, const LbParams & prm, const T * phi,
 		  T * phi_out, const T * u_prev, T * u_next, T * rho, const T * g_in,
-		  T * g_out, const double fzero[3], T * csum, hipStream_t st) {
+		  T * g_out, const double fzero[3], T * csum, const StepPlan & plan, hipStream_t st) {
   const int bz = (g.nz + S::TZ - 1)/S::TZ;
   const int by = (g.ny + S::TY - 1)/S::TY;
-  int xchunk = g.nx;
+  int bx = plan.nchunk;
   if (getenv("LDW_MIN_BLOCKS")) {
     // the fixed rule: halve the chunk until the grid has that many blocks
+    int xchunk = g.nx;
     const int want = tune_min_blocks();
     while (xchunk > 8 && (int64_t) bz*by*((g.nx + xchunk - 1)/xchunk) < want) xchunk = (xchunk + 1)/2;
+    bx = (g.nx + xchunk - 1)/xchunk;
   }
-  else {
-    xchunk = step_xchunk(g.nx, (int64_t) bz*by, resident_slots<T, S>());
-  }
-  const int bx = (g.nx + xchunk - 1)/xchunk;
   const int ntile = bz*by*bx;
   dim3 grid(((ntile + NXCD - 1)/NXCD)*NXCD), block(S::TZ, S::TY, 1);
   const T f0 = T(fzero[0]), f1 = T(fzero[1]), f2 = T(fzero[2]);
   const bool gz = (prm.relax == 0);
 #define L_(O, M, G) hipLaunchKernelGGL((binary_step_kernel<T, S, O, M, G, CONS, GMU>), grid, block, 0, st, \
-				       g, fe, prm, xchunk, bz, by, bx, tune_remap_step(bz*by, ntile), phi, phi_out, u_prev, u_next, rho, \
+				       g, fe, prm, bz, by, bx, tune_remap_step(plan.remap), phi, phi_out, u_prev, u_next, rho, \
 				       g_in, g_out, f0, f1, f2, csum)
 #define L_G(O, M) do { if (gz) L_(O, M, true); else L_(O, M, false); } while (0)
 #define L_M(O) do { if (fe.force_method == 0) L_G(O, 0); else L_G(O, 1); } while (0)
@@ -119,41 +177,35 @@ void launch_shape(const Geom & g, const FeParams & fe, const LbParams & prm, con
 #undef L_
 }
 
-// The block tile: 64 x 4 (z, y) columns (256 threads), or the 512-thread
-// 64 x 8 / 128 x 4 tiles, which halve the share of pulled rows that cross a
-// tile edge in y or z; chosen by precision and lattice size
-// (tune_step_tile).  The tile changes only which block computes a site,
-// not the arithmetic.  With a compensation array (conserve 1), advection
-// order 4 or an external chemical potential gradient the 64 x 8 tile is
-// used, so those kernels are built for one tile only.  The kernels without
-// the external gradient leave its code out, which keeps the FP32 kernels
-// at 3 waves per SIMD.
+// The tile changes only which block computes a site, not the arithmetic.
+// With a compensation array (conserve 1), advection order 4 or an external
+// chemical potential gradient the 64 x 8 tile is used, so those kernels are
+// built for one tile only.  The kernels without the external gradient leave
+// its code out, which keeps the FP32 kernels at 3 waves per SIMD.
 template <typename T>
 void launch(const Geom & g, const FeParams & fe, const LbParams & prm, const T * phi,
 	    T * phi_out, const T * u_prev, T * u_next, T * rho, const T * g_in,
 	    T * g_out, const double fzero[3], T * csum, hipStream_t st) {
-  if (fe.gmu_on) {
-    if (csum) launch_shape<T, Shape<64, 8>, true, true>(g, fe, prm, phi, phi_out, u_prev, u_next, rho, g_in,
-							 g_out, fzero, csum, st);
-    else launch_shape<T, Shape<64, 8>, false, true>(g, fe, prm, phi, phi_out, u_prev, u_next, rho, g_in,
-						    g_out, fzero, nullptr, st);
+  using S64 = Shape<64, 8>;
+  if (fe.gmu_on || csum || fe.order == 4) {
+    const StepPlan n = rounds_plan(g, resident_slots<T, S64>());
+    if (fe.gmu_on && csum) launch_shape<T, S64, true, true>(g, fe, prm, phi, phi_out, u_prev, u_next, rho, g_in,
+							    g_out, fzero, csum, n, st);
+    else if (fe.gmu_on) launch_shape<T, S64, false, true>(g, fe, prm, phi, phi_out, u_prev, u_next, rho, g_in,
+							  g_out, fzero, nullptr, n, st);
+    else if (csum) launch_shape<T, S64, true>(g, fe, prm, phi, phi_out, u_prev, u_next, rho, g_in, g_out, fzero,
+					      csum, n, st);
+    else launch_shape<T, S64, false>(g, fe, prm, phi, phi_out, u_prev, u_next, rho, g_in, g_out, fzero,
+				     nullptr, n, st);
     return;
   }
-  if (csum) {
-    launch_shape<T, Shape<64, 8>, true>(g, fe, prm, phi, phi_out, u_prev, u_next, rho, g_in, g_out, fzero,
-					csum, st);
-    return;
-  }
-  if (fe.order == 4) {
-    launch_shape<T, Shape<64, 8>, false>(g, fe, prm, phi, phi_out, u_prev, u_next, rho, g_in, g_out, fzero,
-					 nullptr, st);
-    return;
-  }
-  switch (tune_step_tile(sizeof(T) == 8 ? 64 : 32, g.nsite)) {
-  case 1: launch_shape<T, Shape<64, 8>, false>(g, fe, prm, phi, phi_out, u_prev, u_next, rho, g_in, g_out, fzero, nullptr, st); break;
-  case 2: launch_shape<T, Shape<128, 4>, false>(g, fe, prm, phi, phi_out, u_prev, u_next, rho, g_in, g_out, fzero, nullptr, st); break;
-  default: launch_shape<T, Shape64x4, false>(g, fe, prm, phi, phi_out, u_prev, u_next, rho, g_in, g_out, fzero, nullptr, st); break;
-  }
+  const StepPlan p = step_plan<T>(g);
+#define TILE_(TZ) launch_shape<T, Shape<TZ, 8>, false>(g, fe, prm, phi, phi_out, u_prev, u_next, rho, g_in, g_out, \
+						       fzero, nullptr, p, st)
+  if (p.tz == 16) TILE_(16);
+  else if (p.tz == 32) TILE_(32);
+  else TILE_(64);
+#undef TILE_
 }
 
 }  // namespace

@@ -20,10 +20,10 @@ namespace ldw {
 namespace tile {
 
 // Tile shape: TZ x TY sites of a plane, one thread per site (block
-// dimensions (TZ, TY)).  The single-lattice step chooses 64 x 4, 64 x 8 or
-// 128 x 4 by precision and lattice size (tune_step_tile); the staged
-// force/Cahn-Hilliard kernel uses 64 x 4; the replica ensemble chooses among
-// several shapes at run time (ensemble.hip).
+// dimensions (TZ, TY)).  The single-lattice step chooses 16 x 8, 32 x 8 or
+// 64 x 8 by precision and lattice (step_plan); the staged force/Cahn-Hilliard
+// kernel uses 64 x 4; the replica ensemble chooses among several shapes at
+// run time (ensemble.hip).
 template <int TZ_, int TY_>
 struct Shape {
   static constexpr int TZ = TZ_, TY = TY_;
@@ -41,11 +41,8 @@ using Shape64x4 = Shape<64, 4>;
 // with its own L2), so physical block k runs on XCD k % 8.  Tiles are
 // numbered z-fastest, then y, then x-chunk.  With remap = 1 XCD g is given
 // the contiguous range of tiles [g*C, (g+1)*C), so tiles that share halo rows
-// and edge cache lines run close together on one L2: that removes about half
-// of the excess L2 fetches, but on MI355X it measured 7% slower at 256^3 than
-// the linear order (remap = 0, the default), whose duplicate edge lines are
-// served by the memory-side Infinity Cache.  Returns false for the padding
-// blocks of the last range.
+// and edge cache lines run close together on one L2.  Returns false for the
+// padding blocks of the last range.
 constexpr int NXCD = 8;
 
 __device__ __forceinline__ bool tile_of_block(int nbz, int nby, int nbx, int remap,

@@ -38,16 +38,18 @@ struct FeParams {
 };
 
 // Launch tuning of the tiled kernels, read once from the environment:
-// LDW_XCD_REMAP (1: XCD-contiguous tile ranges, 0: linear order, default) and
+// LDW_XCD_REMAP (1: XCD-contiguous tile ranges, 0: linear order) and
 // LDW_MIN_BLOCKS (x-chunks are halved until the grid has this many blocks).
+// tune_remap: the staged kernels (linear unless set); tune_remap_step: the
+// single-pass step, `remap` unless set; with tile counts: the Lees-Edwards
+// step's, contiguous where each XCD gets whole x-chunks of ncol column tiles.
 int tune_remap(void);
-// the tile order of the single-lattice step for ncol column tiles and
-// ntile tiles in all (LDW_XCD_REMAP overrides)
+int tune_remap_step(int remap);
 int tune_remap_step(int ncol, int ntile);
 int tune_min_blocks(void);
-// tile of the single-pass step kernel: 0 = 64 x 4, 1 = 64 x 8, 2 = 128 x 4
-// (z x y); LDW_STEP_TILE forces one, else chosen by precision and size
-int tune_step_tile(int precision, int64_t nsite);
+// z extent (16, 32, 64) of the single-pass step's tile that LDW_STEP_TILE
+// (16x8, 32x8, 64x8) forces, else 0: chosen by precision and lattice
+int tune_step_tile(void);
 
 // K1: fused D3Q19 MRT collision + pull propagation.
 //   g_in/g_out: 19 planes of nsite (post-collision distributions; when

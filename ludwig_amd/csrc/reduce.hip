@@ -115,19 +115,18 @@ int tune_remap(void) {
   return v;
 }
 
-int tune_remap_step(int ncol, int ntile) {
+int tune_remap_step(int remap) {
   static int v = -2;
   if (v == -2) {
     const char * e = getenv("LDW_XCD_REMAP");
     v = e ? (atoi(e) ? 1 : 0) : -1;
   }
-  if (v >= 0) return v;
-  // measured on MI355X (binary_step_kernel, FP64, 64 x 8 tiles): the
-  // XCD-contiguous order is 2.5 % faster at 128^3, where each XCD gets
-  // whole x-chunks (32 tiles = every column tile of one chunk), and 7 %
-  // slower at 256^3, where it gets a quarter of a chunk's columns
+  return (v >= 0) ? v : remap;
+}
+
+int tune_remap_step(int ncol, int ntile) {
   const int per = (ntile + 7)/8;
-  return (ntile % 8 == 0 && per % ncol == 0) ? 1 : 0;
+  return tune_remap_step((ntile % 8 == 0 && per % ncol == 0) ? 1 : 0);
 }
 
 int tune_min_blocks(void) {
@@ -136,22 +135,16 @@ int tune_min_blocks(void) {
   return v;
 }
 
-int tune_step_tile(int precision, int64_t nsite) {
-  static int v = -2;
-  if (v == -2) {
+int tune_step_tile(void) {
+  static int v = -1;
+  if (v < 0) {
     const char * e = getenv("LDW_STEP_TILE");
-    v = -1;
-    if (e && strcmp(e, "64x4") == 0) v = 0;
-    else if (e && strcmp(e, "64x8") == 0) v = 1;
-    else if (e && strcmp(e, "128x4") == 0) v = 2;
+    v = 0;
+    if (e && strcmp(e, "16x8") == 0) v = 16;
+    else if (e && strcmp(e, "32x8") == 0) v = 32;
+    else if (e && strcmp(e, "64x8") == 0) v = 64;
   }
-  if (v >= 0) return v;
-  // measured on MI355X (C2 physics, planes per block from the launch cost
-  // model): FP64 is fastest with 64 x 8 tiles at 128^3 and 256^3; FP32 with
-  // 128 x 4 tiles up to 128^3 and with 64 x 8 tiles at 256^3 (660 us
-  // against 686 us for 64 x 4)
-  if (precision == 64) return 1;
-  return (nsite <= ((int64_t) 1 << 22)) ? 2 : 1;
+  return v;
 }
 
 int sum_blocks(int64_t n) {

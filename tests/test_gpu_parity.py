@@ -469,3 +469,25 @@ def test_fused_and_unfused_force_paths_agree():
     assert_exact(b1.hydro_fields()[2], b2.hydro_fields()[2], "force")
     b1.close()
     b2.close()
+
+
+# The single-pass step's tiles and chunks: 16, 32 and 64 wide rows, one plane
+# per block and several, columns and planes that the tile and the chunks cut
+# unevenly, lattices smaller than a tile, too many columns for one round of
+# blocks, and the large-lattice rule (rows of 32, chunks of 3 planes)
+@pytest.mark.parametrize("shape", [(3, 5, 4), (7, 9, 15), (50, 17, 30), (12, 16, 33), (61, 40, 70), (3, 512, 272),
+                                   (20, 203, 204)])
+def test_step_tiles_match_oracle(shape):
+    p = dict(a=-0.0625, b=0.0625, kappa=0.04, mobility=0.25)
+    nsteps = 3
+    print(f"step tiles {shape}", flush=True)
+    b = L.BinaryFluid(shape, tau=1.0, fatal=True, **p)
+    b.init_spinodal(77, 0.05, 0.1)
+    b.step(nsteps)
+    got = (b.f(), b.phi_field()) + b.hydro_fields()[:2]
+    b.close()
+    f0 = O.equilibrium(shape, rho_uniform=1.0)
+    phi0 = O.spinodal(shape, 77, 0.05, 0.1)
+    want = O.binary_steps(shape, nsteps, O.lb_param(tau=1.0), O.fe_param(**p), f0, phi0)
+    for name, g, w in zip(("f", "phi", "rho", "u"), got, want):
+        assert np.array_equal(g, w), name
