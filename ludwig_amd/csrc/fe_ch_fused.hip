@@ -1,7 +1,7 @@
 // fe_ch_fused.hip -- K23: thermodynamic force and Cahn-Hilliard update of
 // the symmetric free energy in one pass over phi.
 //
-// One block owns a TY x TZ tile of (y, z) columns and marches along x.  LDS
+// One block owns a TY x TZ (8 x 16) tile of (y, z) columns and marches along x.  LDS
 // holds a ring of 5 phi planes with a halo of 2 in y and z, and a ring of 3
 // planes of Q = (d_x phi, d_y phi, d_z phi, p0, mu) with a halo of 1, so
 // every phi value is fetched from memory about once and every stencil
@@ -29,11 +29,10 @@ namespace ldw {
 namespace {
 
 using namespace tile;
-using S = Shape64x4;
 
-template <typename T, int ORDER, int METHOD, bool HAVE_U>
+template <typename T, class S, int ORDER, int METHOD, bool HAVE_U>
 __global__ void __launch_bounds__(S::NT)
-force_ch_kernel(Geom g, FeParams fe, int xchunk, int nbz, int nby, int nbx, int remap, const T * __restrict__ phi,
+force_ch_kernel(Geom g, FeParams fe, int nbz, int nby, int nbx, int remap, const T * __restrict__ phi,
 		const T * __restrict__ u, T * __restrict__ force, T * __restrict__ phi_out,
 		T * __restrict__ csum, int force_mode, T fz0, T fz1, T fz2) {
 
@@ -43,8 +42,10 @@ force_ch_kernel(Geom g, FeParams fe, int xchunk, int nbz, int nby, int nbx, int 
   if (!tile_of_block(nbz, nby, nbx, remap, bzi, byi, bxi)) return;
   const int tz = threadIdx.x, ty = threadIdx.y;
   const int z0 = bzi*S::TZ, y0 = byi*S::TY;
-  const int xb = bxi*xchunk;
-  const int xe = min(xb + xchunk, g.nx);
+  // nbx chunks of planes, even to within one plane
+  const int xq = g.nx/nbx, xr = g.nx - xq*nbx;
+  const int xb = bxi*xq + min(bxi, xr);
+  const int xe = xb + xq + (bxi < xr ? 1 : 0);
   const int y = y0 + ty, z = z0 + tz;
   const bool active = (y < g.ny) && (z < g.nz);
 
@@ -99,21 +100,16 @@ force_ch_kernel(Geom g, FeParams fe, int xchunk, int nbz, int nby, int nbx, int 
   }
 }
 
-template <typename T>
-void launch(const Geom & g, const FeParams & fe, const T * phi, const T * u, T * force,
-	    T * phi_out, T * csum, int force_mode, const double fzero[3], hipStream_t st) {
+template <typename T, class S>
+void launch_shape(const Geom & g, const FeParams & fe, const T * phi, const T * u, T * force,
+		  T * phi_out, T * csum, int force_mode, const double fzero[3], int bx, hipStream_t st) {
   const int bz = (g.nz + S::TZ - 1)/S::TZ;
   const int by = (g.ny + S::TY - 1)/S::TY;
-  // enough blocks to fill 256 CUs several times; chunk of x planes per block
-  int xchunk = g.nx;
-  const int want = tune_min_blocks();
-  while (xchunk > 8 && (int64_t) bz*by*((g.nx + xchunk - 1)/xchunk) < want) xchunk = (xchunk + 1)/2;
-  const int bx = (g.nx + xchunk - 1)/xchunk;
   const int ntile = bz*by*bx;
   dim3 grid(((ntile + NXCD - 1)/NXCD)*NXCD), block(S::TZ, S::TY, 1);
   const T f0 = T(fzero[0]), f1 = T(fzero[1]), f2 = T(fzero[2]);
-#define L_(O, M, U) hipLaunchKernelGGL((force_ch_kernel<T, O, M, U>), grid, block, 0, st, \
-				       g, fe, xchunk, bz, by, bx, tune_remap(), phi, u, force, phi_out, csum, force_mode, \
+#define L_(O, M, U) hipLaunchKernelGGL((force_ch_kernel<T, S, O, M, U>), grid, block, 0, st, \
+				       g, fe, bz, by, bx, tune_remap(), phi, u, force, phi_out, csum, force_mode, \
 				       f0, f1, f2)
 #define L_U(O, M) do { if (u) L_(O, M, true); else L_(O, M, false); } while (0)
 #define L_M(O) do { if (fe.force_method == 0) L_U(O, 0); else L_U(O, 1); } while (0)
@@ -124,6 +120,42 @@ void launch(const Geom & g, const FeParams & fe, const T * phi, const T * u, T *
 #undef L_M
 #undef L_U
 #undef L_
+}
+
+// Tile and chunks: 16 x 8 tiles in one round of as many blocks as the GPU
+// holds (5 per CU in FP64).  The pass reads and writes little, so it is bound
+// by the length of a block (prologue and planes in a row), not by memory.
+// us at 100x84x76 / 128^3 / 144^3 FP64: 26 / 57 / 79, against 47 / 73 / 149 for 64 x
+// 4 tiles in 2048 blocks (the second round of which repeats the prologue) and
+// 33 / 65 / 84 for 32 x 8 tiles at their best; FP32 21 / 40 / 54 against 27 / 45 / 88.
+using S16 = Shape<16, 8>;
+
+template <typename T>
+int resident_slots() {
+  static int slots = 0;
+  if (slots == 0) {
+    int per_cu = 0, dev = 0;
+    hipDeviceProp_t prop;
+    if (hipGetDevice(&dev) != hipSuccess || hipGetDeviceProperties(&prop, dev) != hipSuccess
+	|| hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, force_ch_kernel<T, S16, 1, 0, true>, S16::NT, 0)
+	   != hipSuccess || per_cu < 1) {
+      (void) hipGetLastError();
+      return 1024;
+    }
+    slots = per_cu*prop.multiProcessorCount;
+  }
+  return slots;
+}
+
+template <typename T>
+void launch(const Geom & g, const FeParams & fe, const T * phi, const T * u, T * force,
+	    T * phi_out, T * csum, int force_mode, const double fzero[3], hipStream_t st) {
+  const int64_t ncol = (int64_t) ((g.nz + 15)/16)*((g.ny + 7)/8);
+  // more columns than slots: chunks of 16 planes
+  int64_t bx = resident_slots<T>()/ncol;
+  if (bx < 1) bx = (g.nx + 15)/16;
+  if (bx > g.nx) bx = g.nx;
+  launch_shape<T, S16>(g, fe, phi, u, force, phi_out, csum, force_mode, fzero, (int) bx, st);
 }
 
 }  // namespace

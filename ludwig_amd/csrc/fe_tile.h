@@ -22,7 +22,7 @@ namespace tile {
 // Tile shape: TZ x TY sites of a plane, one thread per site (block
 // dimensions (TZ, TY)).  The single-lattice step chooses 16 x 8, 32 x 8 or
 // 64 x 8 by precision and lattice (step_plan); the staged force/Cahn-Hilliard
-// kernel uses 64 x 4; the replica ensemble chooses among several shapes at
+// kernel uses 16 x 8; the replica ensemble chooses among several shapes at
 // run time (ensemble.hip).
 template <int TZ_, int TY_>
 struct Shape {
@@ -34,8 +34,6 @@ struct Shape {
   static constexpr int QPLANE = QZ*QY;
   static constexpr int NPRE = (PPLANE + NT - 1)/NT;   // phi values prefetched per thread
 };
-
-using Shape64x4 = Shape<64, 4>;
 
 // Tile order.  Workgroups are dispatched round-robin over the 8 XCDs (each
 // with its own L2), so physical block k runs on XCD k % 8.  Tiles are

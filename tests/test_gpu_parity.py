@@ -474,8 +474,9 @@ def test_fused_and_unfused_force_paths_agree():
 # The single-pass step's tiles and chunks: 16, 32 and 64 wide rows, one plane
 # per block and several, columns and planes that the tile and the chunks cut
 # unevenly, lattices smaller than a tile, too many columns for one round of
-# blocks, and the large-lattice rule (rows of 32, chunks of 3 planes)
-@pytest.mark.parametrize("shape", [(3, 5, 4), (7, 9, 15), (50, 17, 30), (12, 16, 33), (61, 40, 70), (3, 512, 272),
+# blocks of either kernel (the first step is staged), and the large-lattice rule
+# (rows of 32, chunks of 3 planes)
+@pytest.mark.parametrize("shape", [(3, 5, 4), (7, 9, 15), (50, 17, 30), (12, 16, 33), (61, 40, 70), (3, 512, 340),
                                    (20, 203, 204)])
 def test_step_tiles_match_oracle(shape):
     p = dict(a=-0.0625, b=0.0625, kappa=0.04, mobility=0.25)
