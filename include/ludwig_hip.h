@@ -629,6 +629,20 @@ int ldw_conv3d_weights_prep(const float * w, void * wf, void * wd, int cin, int 
 /* Elementwise and reshaping kernels of the network (device pointers) */
 int ldw_nn_silu_fwd(const float * z, void * a, long long n);
 int ldw_nn_silu_bwd(const float * z, const float * da, float * dz, void * dzb, long long n);
+/* SiLU backward and bias gradient in one pass: dz = da silu'(z), dzb = bf16(dz),
+ * db[ch] = the sum of dz over the positions (nx, ny, nz: the lattice of z;
+ * c channels, a multiple of 4 up to 1024, arrays 16-byte aligned).  da is
+ *   given                                            (ldw_nn_silu_bwd_bias)
+ *   columns off .. off+c of dcat[p][ccat] + dpool[pooled p]/8   (.._skip)
+ *   the sum over p's 8 fine children of columns 0 .. c of
+ *   dcat[child][ccat]                                            (.._up)
+ * i.e. what ldw_nn_split, _pool2_bwd (added) and _up2_bwd would form. */
+int ldw_nn_silu_bwd_bias(const float * z, const float * da, void * dzb, float * db, int batch, int nx,
+			 int ny, int nz, int c);
+int ldw_nn_silu_bwd_bias_skip(const float * z, const float * dcat, int ccat, int off, const float * dpool,
+			      void * dzb, float * db, int batch, int nx, int ny, int nz, int c);
+int ldw_nn_silu_bwd_bias_up(const float * z, const float * dcat, int ccat, void * dzb, float * db, int batch,
+			    int nx, int ny, int nz, int c);
 int ldw_nn_bias_grad(const float * dz, float * db, long long npos, int c, int accumulate);
 int ldw_nn_pool2_fwd(const void * in, void * out, int batch, int nx, int ny, int nz, int c);
 int ldw_nn_pool2_bwd(const float * dout, float * din, int batch, int nx, int ny, int nz, int c,

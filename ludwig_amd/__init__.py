@@ -186,6 +186,9 @@ def lib():
         "ldw_conv3d_weights_prep": [vp, vp, vp, ctypes.c_int, ctypes.c_int],
         "ldw_nn_silu_fwd": [vp, vp, ctypes.c_longlong],
         "ldw_nn_silu_bwd": [vp, vp, vp, vp, ctypes.c_longlong],
+        "ldw_nn_silu_bwd_bias": [vp] * 4 + [ctypes.c_int] * 5,
+        "ldw_nn_silu_bwd_bias_skip": [vp, vp, ctypes.c_int, ctypes.c_int, vp, vp, vp] + [ctypes.c_int] * 5,
+        "ldw_nn_silu_bwd_bias_up": [vp, vp, ctypes.c_int, vp, vp] + [ctypes.c_int] * 5,
         "ldw_nn_bias_grad": [vp, vp, ctypes.c_longlong, ctypes.c_int, ctypes.c_int],
         "ldw_nn_pool2_fwd": [vp, vp] + [ctypes.c_int] * 5,
         "ldw_nn_pool2_bwd": [vp, vp] + [ctypes.c_int] * 6,

@@ -201,6 +201,13 @@ hipError_t nn_silu_bwd(const float * z, const float * da, float * dz, uint16_t *
 int64_t nn_bias_grad_workspace(int64_t npos, int c);
 hipError_t nn_bias_grad(const float * dz, float * db, float * work, int64_t npos, int c,
 			int accumulate, hipStream_t s);
+// SiLU backward and bias gradient in one pass, the incoming gradient gathered
+// (mode 0 plain, 1 skip branch, 2 below an upsampling; nn_ops.hip); c, ld, off
+// multiples of 4, c at most 1024, arrays 16-byte (dzb 8-byte) aligned
+int64_t nn_silu_bwd_sums_workspace(int c);
+hipError_t nn_silu_bwd_sums(int mode, const float * z, const float * d1, const float * d2, uint16_t * dzb,
+			    float * db, float * work, int batch, int nx, int ny, int nz, int c, int ld, int off,
+			    hipStream_t s);
 hipError_t nn_pool2_fwd(const uint16_t * in, uint16_t * out, int batch, int nx, int ny, int nz, int c,
 			hipStream_t s);
 hipError_t nn_pool2_bwd(const float * dout, float * din, int batch, int nx, int ny, int nz, int c,

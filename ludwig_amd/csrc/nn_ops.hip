@@ -141,6 +141,81 @@ sum_rows_kernel(const float * __restrict__ part, float * __restrict__ out, int n
   }
 }
 
+// SiLU backward of one layer with its bias gradient, the incoming gradient da
+// gathered from where the network's backward pass leaves it:
+//   DA_PLAIN  da[p][c];
+//   DA_SKIP   the skip branch: columns off .. off + c of the concatenation's
+//             gradient d1[p][ld], plus an eighth of the pooled position's
+//             gradient d2[parent][c];
+//   DA_UP     the branch below an upsampling: the sum over the 8 fine
+//             children of columns 0 .. c of d1[child][ld].
+// Writes dzb = bf16(dz) and the blocks' partial sums of dz (FP32) over the
+// positions.  The gradient dz itself, the split and the unpooled gradients
+// never go to memory: 10 to 14 bytes a value where the separate passes (split,
+// unpool, SiLU, bias) move 30 to 46.  A thread has 4 channels; a block goes
+// through z lines of the lattice, `rows` positions at a time, so that the
+// parent and child positions take no division per value.
+enum { DA_PLAIN, DA_SKIP, DA_UP };
+
+template <int MODE>
+__global__ void __launch_bounds__(256)
+silu_bwd_sums_kernel(const float * __restrict__ z, const float * __restrict__ d1, const float * __restrict__ d2,
+		     uint16_t * __restrict__ dzb, float * __restrict__ part, int64_t nline, int nx, int ny, int nz,
+		     int c, int ld, int off) {
+  __shared__ float sh[256*4];
+  const int tr = c/4, rows = 256/tr;
+  const int row = threadIdx.x/tr, ch = 4*(threadIdx.x%tr);
+  float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (row < rows) {
+    for (int64_t l = blockIdx.x; l < nline; l += gridDim.x) {
+      // line (b, x, y): uniform over the block
+      int64_t other = 0;
+      if constexpr (MODE != DA_PLAIN) {
+	const int y = (int) (l % ny), x = (int) ((l/ny) % nx);
+	const int64_t b = l/((int64_t) nx*ny);
+	if constexpr (MODE == DA_SKIP) other = ((b*(nx/2) + x/2)*(ny/2) + y/2)*(nz/2);
+	else other = ((b*2*nx + 2*x)*2*ny + 2*y)*2*nz;
+      }
+      for (int k = row; k < nz; k += rows) {
+	const int64_t p = l*nz + k;
+	const float4 v = *reinterpret_cast<const float4 *>(z + p*c + ch);
+	float4 d;
+	if constexpr (MODE == DA_PLAIN) {
+	  d = *reinterpret_cast<const float4 *>(d1 + p*c + ch);
+	}
+	else if constexpr (MODE == DA_SKIP) {
+	  d = *reinterpret_cast<const float4 *>(d1 + p*ld + off + ch);
+	  const float4 e = *reinterpret_cast<const float4 *>(d2 + (other + k/2)*c + ch);
+	  d.x += 0.125f*e.x; d.y += 0.125f*e.y; d.z += 0.125f*e.z; d.w += 0.125f*e.w;
+	}
+	else {
+	  d = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+	  for (int j = 0; j < 8; j++) {
+	    const int64_t f = other + ((int64_t) (j >> 2)*2*ny + ((j >> 1) & 1))*2*nz + 2*k + (j & 1);
+	    const float4 e = *reinterpret_cast<const float4 *>(d1 + f*ld + ch);
+	    d.x += e.x; d.y += e.y; d.z += e.z; d.w += e.w;
+	  }
+	}
+	const float4 g = make_float4(silu_grad(v.x, d.x), silu_grad(v.y, d.y), silu_grad(v.z, d.z), silu_grad(v.w, d.w));
+	*reinterpret_cast<uint2 *>(dzb + p*c + ch) = bf16x4(g);
+	s[0] += g.x; s[1] += g.y; s[2] += g.z; s[3] += g.w;
+      }
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 4; k++) sh[4*threadIdx.x + k] = s[k];
+  __syncthreads();
+  if (row == 0) {
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      float t = s[k];
+      for (int j = 1; j < rows; j++) t += sh[4*(threadIdx.x + j*tr) + k];
+      part[(int64_t) blockIdx.x*c + ch + k] = t;
+    }
+  }
+}
+
 // coarse (nx/2, ny/2, nz/2) = mean of the 8 fine children
 __global__ void pool2_fwd_kernel(const uint16_t * __restrict__ in, uint16_t * __restrict__ out,
 				 int batch, int nx, int ny, int nz, int c) {
@@ -527,6 +602,23 @@ hipError_t nn_bias_grad(const float * dz, float * db, float * work, int64_t npos
   launch_sum_rows(work, db, (int) nblk, c, accumulate, s);
   return hipGetLastError();
 }
+
+hipError_t nn_silu_bwd_sums(int mode, const float * z, const float * d1, const float * d2, uint16_t * dzb,
+			    float * db, float * work, int batch, int nx, int ny, int nz, int c, int ld, int off,
+			    hipStream_t s) {
+  const int64_t nline = (int64_t) batch*nx*ny;
+  const int nblk = (int) (nline < 2*SUM_ROWS ? nline : 2*SUM_ROWS);
+#define SUMS_(MODE) hipLaunchKernelGGL(silu_bwd_sums_kernel<MODE>, dim3(nblk), dim3(256), 0, s, z, d1, d2, dzb, work, \
+				       nline, nx, ny, nz, c, ld, off)
+  if (mode == DA_PLAIN) SUMS_(DA_PLAIN);
+  else if (mode == DA_SKIP) SUMS_(DA_SKIP);
+  else SUMS_(DA_UP);
+#undef SUMS_
+  launch_sum_rows(work, db, nblk, c, 0, s);
+  return hipGetLastError();
+}
+
+int64_t nn_silu_bwd_sums_workspace(int c) { return (int64_t) 2*SUM_ROWS*c; }
 
 hipError_t nn_pool2_fwd(const uint16_t * in, uint16_t * out, int batch, int nx, int ny, int nz, int c,
 			hipStream_t s) {

@@ -165,6 +165,38 @@ extern "C" int ldw_nn_bias_grad(const float * dz, float * db, long long npos, in
   return 0;
 }
 
+static int silu_bwd_sums(const char * who, int mode, const float * z, const float * d1, const float * d2, void * dzb,
+			 float * db, int batch, int nx, int ny, int nz, int c, int ld, int off) {
+  READY();
+  if (!z || !d1 || !dzb || !db || (mode == 1 && !d2)) LDW_FAIL("%s: null buffer", who);
+  if (batch < 1 || nx < 1 || ny < 1 || nz < 1) LDW_FAIL("%s: bad sizes %d x %d x %d x %d", who, batch, nx, ny, nz);
+  if (c < 4 || c > 1024 || c % 4 || ld % 4 || off % 4 || off < 0 || off + c > ld)
+    LDW_FAIL("%s: channels %d of %d at %d (multiples of 4, at most 1024)", who, c, ld, off);
+  if (mode == 1 && (nx % 2 || ny % 2 || nz % 2)) LDW_FAIL("%s: odd lattice %d x %d x %d", who, nx, ny, nz);
+  if ((((uintptr_t) z | (uintptr_t) d1 | (uintptr_t) d2) % 16) || ((uintptr_t) dzb % 8))
+    LDW_FAIL("%s: arrays must be 16-byte aligned (the BF16 one 8-byte)", who);
+  void * work = nullptr;
+  if (scratch_buffer(g_bias, (size_t) ldw::nn_silu_bwd_sums_workspace(c)*sizeof(float), &work)) return -1;
+  KCHECK(ldw::nn_silu_bwd_sums(mode, z, d1, d2, (uint16_t *) dzb, db, (float *) work, batch, nx, ny, nz, c, ld, off,
+			       ldw::api::stream()));
+  return 0;
+}
+
+extern "C" int ldw_nn_silu_bwd_bias(const float * z, const float * da, void * dzb, float * db, int batch, int nx,
+				    int ny, int nz, int c) {
+  return silu_bwd_sums("ldw_nn_silu_bwd_bias", 0, z, da, nullptr, dzb, db, batch, nx, ny, nz, c, c, 0);
+}
+
+extern "C" int ldw_nn_silu_bwd_bias_skip(const float * z, const float * dcat, int ccat, int off, const float * dpool,
+					 void * dzb, float * db, int batch, int nx, int ny, int nz, int c) {
+  return silu_bwd_sums("ldw_nn_silu_bwd_bias_skip", 1, z, dcat, dpool, dzb, db, batch, nx, ny, nz, c, ccat, off);
+}
+
+extern "C" int ldw_nn_silu_bwd_bias_up(const float * z, const float * dcat, int ccat, void * dzb, float * db, int batch,
+				       int nx, int ny, int nz, int c) {
+  return silu_bwd_sums("ldw_nn_silu_bwd_bias_up", 2, z, dcat, nullptr, dzb, db, batch, nx, ny, nz, c, ccat, 0);
+}
+
 extern "C" int ldw_nn_pool2_fwd(const void * in, void * out, int batch, int nx, int ny, int nz, int c) {
   READY();
   if (nx % 2 || ny % 2 || nz % 2) LDW_FAIL("ldw_nn_pool2_fwd: odd lattice %d x %d x %d", nx, ny, nz);

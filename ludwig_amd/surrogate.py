@@ -222,14 +222,13 @@ class UNet:
             b["z_" + name] = DeviceArray(p * co, np.float32)
             if name != "out":
                 b["a_" + name] = DeviceArray(p * co, np.uint16)
+                b["dzb_" + name] = DeviceArray(p * co, np.uint16)
+            if name in ("e0a", "e1a", "e2a", "b0", "d0"):
                 b["da_" + name] = DeviceArray(p * co, np.float32)
-            b["dz_" + name] = DeviceArray(p * co, np.float32)
-            b["dzb_" + name] = DeviceArray(p * co, np.uint16)
         for l, c in ((1, C[0]), (2, C[1]), (3, C[2])):
             b[f"pool{l}"] = DeviceArray(P[l] * c, np.uint16)
             b[f"dpool{l}"] = DeviceArray(P[l] * c, np.float32)
         for l, c_up, c_skip in ((2, C[3], C[2]), (1, C[2], C[1]), (0, C[1], C[0])):
-            b[f"dup{l}"] = DeviceArray(P[l] * c_up, np.float32)
             b[f"cat{l}"] = DeviceArray(P[l] * (c_up + c_skip), np.uint16)
             b[f"dcat{l}"] = DeviceArray(P[l] * (c_up + c_skip), np.float32)
         self._bufs[key] = b
@@ -278,55 +277,58 @@ class UNet:
         self._last = b
         return b["z_out"]
 
-    def _conv_back(self, b, name, x, dzb, dz, dx=None, acc_dx=0):
-        """Weight and bias gradients of layer `name`; input gradient into dx."""
+    def _conv_back(self, b, name, x, dzb, dx=None):
+        """Weight gradient of layer `name`; input gradient into dx."""
         L = lib()
         _, ci, co = self.layout[name]
-        l = LEVEL[name]
-        nx, ny, nz = b["shape"][l]
+        nx, ny, nz = b["shape"][LEVEL[name]]
         batch = b["batch"]
         _ck(L.ldw_conv3d_bwd_weight(_v(x), _v(dzb), self.wptr(name, self.g), batch, nx, ny, nz, ci, co, 0),
             f"wgrad {name}")
-        _ck(L.ldw_nn_bias_grad(_v(dz), self.bptr(name, self.g), b["P"][l], co, 0), f"bias grad {name}")
         if dx is not None:
-            _ck(L.ldw_conv3d_bwd_data(_v(dzb), _v(self.wd[name]), _v(dx), batch, nx, ny, nz, ci, co, acc_dx),
+            _ck(L.ldw_conv3d_bwd_data(_v(dzb), _v(self.wd[name]), _v(dx), batch, nx, ny, nz, ci, co, 0),
                 f"dgrad {name}")
 
-    def _act_back(self, b, name):
+    def _act_back(self, b, name, up=None, skip=None):
+        """SiLU backward of layer `name` into its dzb, and its bias gradient.
+        The incoming gradient is da_<name>; with `up` the upsampled branch of
+        that level's concatenation, with `skip` the skip branch of that
+        level's concatenation plus the pooled branch's gradient."""
         L = lib()
         co = self.layout[name][2]
-        _ck(L.ldw_nn_silu_bwd(_v(b["z_" + name]), _v(b["da_" + name]), _v(b["dz_" + name]),
-                              _v(b["dzb_" + name]), b["P"][LEVEL[name]] * co), f"silu back {name}")
+        out = (_v(b["dzb_" + name]), self.bptr(name, self.g), b["batch"], *b["shape"][LEVEL[name]], co)
+        z = _v(b["z_" + name])
+        if up is not None:
+            dcat = b[f"dcat{up}"]
+            _ck(L.ldw_nn_silu_bwd_bias_up(z, _v(dcat), dcat.n // b["P"][up], *out), f"silu back {name}")
+        elif skip is not None:
+            dcat = b[f"dcat{skip}"]
+            ccat = dcat.n // b["P"][skip]
+            _ck(L.ldw_nn_silu_bwd_bias_skip(z, _v(dcat), ccat, ccat - co, _v(b[f"dpool{skip + 1}"]), *out),
+                f"silu back {name}")
+        else:
+            _ck(L.ldw_nn_silu_bwd_bias(z, _v(b["da_" + name]), *out), f"silu back {name}")
 
     def backward(self, dyb, dyf):
         """Gradients of the loss into self.g, from the output gradient dyb
         (BF16) and dyf (FP32), both [batch*nsite][16]."""
-        L = lib()
         b = self._last
         if not b["keep"]:
             raise RuntimeError("backward after an inference-only forward pass")
-        batch, sh, P = b["batch"], b["shape"], b["P"]
-        self._conv_back(b, "out", b["a_d0"], dyb, dyf, b["da_d0"])
-        for l, low, skip, name in ((0, "d1", "e0b", "d0"), (1, "d2", "e1b", "d1"), (2, "b1", "e2b", "d2")):
-            cu, cs = self.layout[low][2], self.layout[skip][2]
-            self._act_back(b, name)
-            self._conv_back(b, name, b[f"cat{l}"], b["dzb_" + name], b["dz_" + name], b[f"dcat{l}"])
-            # the skip branch's gradient is written first; pooling adds to it later
-            _ck(L.ldw_nn_split(_v(b[f"dcat{l}"]), cu, cs, _v(b[f"dup{l}"]), _v(b["da_" + skip]), P[l], 0, 0),
-                "split")
-            _ck(L.ldw_nn_up2_bwd(_v(b[f"dup{l}"]), _v(b["da_" + low]), batch, *sh[l + 1], cu), "up back")
-        for l, prev, na, nb in ((3, "e2b", "b0", "b1"), (2, "e1b", "e2a", "e2b"), (1, "e0b", "e1a", "e1b")):
-            self._act_back(b, nb)
-            self._conv_back(b, nb, b["a_" + na], b["dzb_" + nb], b["dz_" + nb], b["da_" + na])
+        self._conv_back(b, "out", b["a_d0"], dyb, b["da_d0"])
+        _ck(lib().ldw_nn_bias_grad(_v(dyf), self.bptr("out", self.g), b["P"][0], COUT, 0), "bias grad out")
+        for l, name, up in ((0, "d0", None), (1, "d1", 0), (2, "d2", 1)):
+            self._act_back(b, name, up=up)
+            self._conv_back(b, name, b[f"cat{l}"], b["dzb_" + name], b[f"dcat{l}"])
+        for l, na, nb in ((3, "b0", "b1"), (2, "e2a", "e2b"), (1, "e1a", "e1b")):
+            self._act_back(b, nb, **(dict(up=2) if l == 3 else dict(skip=l)))
+            self._conv_back(b, nb, b["a_" + na], b["dzb_" + nb], b["da_" + na])
             self._act_back(b, na)
-            self._conv_back(b, na, b[f"pool{l}"], b["dzb_" + na], b["dz_" + na], b[f"dpool{l}"])
-            c = self.layout[prev][2]
-            _ck(L.ldw_nn_pool2_bwd(_v(b[f"dpool{l}"]), _v(b["da_" + prev]), batch, *sh[l - 1], c, 1),
-                "pool back")
-        self._act_back(b, "e0b")
-        self._conv_back(b, "e0b", b["a_e0a"], b["dzb_e0b"], b["dz_e0b"], b["da_e0a"])
+            self._conv_back(b, na, b[f"pool{l}"], b["dzb_" + na], b[f"dpool{l}"])
+        self._act_back(b, "e0b", skip=0)
+        self._conv_back(b, "e0b", b["a_e0a"], b["dzb_e0b"], b["da_e0a"])
         self._act_back(b, "e0a")
-        self._conv_back(b, "e0a", b["x"], b["dzb_e0a"], b["dz_e0a"], None)
+        self._conv_back(b, "e0a", b["x"], b["dzb_e0a"])
 
 
 class Normaliser:

@@ -191,6 +191,36 @@ def test_silu_backward_vector_path_is_the_scalar_one(n):
     assert np.allclose(out[0][0], da * sg * (1 + zz * (1 - sg)), rtol=1e-5, atol=1e-6)
 
 
+# the one-pass backward against the passes it stands for, bit for bit, and the
+# bias gradient against float64: fewer and more positions than a block covers,
+# channel counts that leave threads idle, more lines than blocks
+@pytest.mark.parametrize("batch,shape,c,other", [(1, (2, 2, 2), 4, 8), (2, (4, 6, 10), 48, 64), (1, (2, 4, 34), 1024, 4),
+                                                 (3, (34, 28, 4), 32, 48)])
+def test_silu_backward_bias_one_pass(batch, shape, c, other):
+    lib = L.lib()
+    rng = np.random.default_rng(c)
+    nx, ny, nz = shape
+    n, nf, nc = (batch * int(np.prod([s * k // 2 for s in shape])) for k in (2, 4, 1))
+    f32 = lambda k: dev(rng.standard_normal(k).astype(np.float32), np.float32)
+    z, da, dcat, dpool, dfine = f32(n * c), f32(n * c), f32(n * (other + c)), f32(nc * c), f32(nf * (c + other))
+    skip, up, rest = (L.DeviceArray(k, np.float32) for k in (n * c, nf * c, nf * (c + other)))
+    assert lib.ldw_nn_split(vp(dcat), other, c, None, vp(skip), n, 0, 0) == 0
+    assert lib.ldw_nn_pool2_bwd(vp(dpool), vp(skip), batch, nx, ny, nz, c, 1) == 0
+    assert lib.ldw_nn_split(vp(dfine), c, other, vp(up), None, nf, 0, 0) == 0
+    assert lib.ldw_nn_up2_bwd(vp(up), vp(rest), batch, nx, ny, nz, c) == 0
+    dz, db = L.DeviceArray(n * c, np.float32), L.DeviceArray(c, np.float32)
+    want_b, got_b = L.DeviceArray(n * c, np.uint16), L.DeviceArray(n * c, np.uint16)
+    at_ = (vp(got_b), vp(db), batch, nx, ny, nz, c)
+    for src, call in ((da, lambda: lib.ldw_nn_silu_bwd_bias(vp(z), vp(da), *at_)),
+                      (skip, lambda: lib.ldw_nn_silu_bwd_bias_skip(vp(z), vp(dcat), other + c, other, vp(dpool), *at_)),
+                      (rest, lambda: lib.ldw_nn_silu_bwd_bias_up(vp(z), vp(dfine), c + other, *at_))):
+        assert lib.ldw_nn_silu_bwd(vp(z), vp(src), vp(dz), vp(want_b), n * c) == 0
+        assert call() == 0
+        assert np.array_equal(got_b.download(), want_b.download())
+        g = dz.download().reshape(n, c).astype(np.float64)
+        within(db.download().astype(np.float64), g.sum(0), 2 * (n + 1) * EPS32 * np.abs(g).sum(0) + 1e-30, "bias")
+
+
 def test_pool_up_concat_split_silu_exact():
     lib = L.lib()
     rng = np.random.default_rng(1)
