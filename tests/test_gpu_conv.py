@@ -191,6 +191,26 @@ def test_silu_backward_vector_path_is_the_scalar_one(n):
     assert np.allclose(out[0][0], da * sg * (1 + zz * (1 - sg)), rtol=1e-5, atol=1e-6)
 
 
+# 8 channels at a time or singly (odd counts of 8, off = 1: misaligned), against
+# float64 and each other
+@pytest.mark.parametrize("batch,shape,c", [(1, (2, 2, 2), 8), (2, (4, 6, 10), 40), (3, (2, 130, 66), 16)])
+def test_pool_vector_path_is_the_scalar_one(batch, shape, c):
+    lib = L.lib()
+    rng = np.random.default_rng(c)
+    n = batch * int(np.prod(shape)) * c
+    a = bf16_round(rng.standard_normal(n))
+    out = []
+    for off in (0, 1):
+        d = dev(np.concatenate([np.zeros(off, np.uint16), bf16_bits(a)]), np.uint16)
+        o = L.DeviceArray(n // 8 + off, np.uint16)
+        assert lib.ldw_nn_pool2_fwd(at(d, 2 * off), at(o, 2 * off), batch, *shape, c) == 0
+        out.append(o.download()[off:])
+    assert np.array_equal(out[0], out[1])
+    nx, ny, nz = shape
+    want = a.astype(np.float64).reshape(batch, nx // 2, 2, ny // 2, 2, nz // 2, 2, c).mean(axis=(2, 4, 6)).ravel()
+    assert np.allclose(bf16_value(out[0]), want, rtol=2 ** -8, atol=1e-6)
+
+
 # the one-pass backward against the passes it stands for, bit for bit, and the
 # bias gradient against float64: fewer and more positions than a block covers,
 # channel counts that leave threads idle, more lines than blocks
