@@ -268,10 +268,10 @@ conv3_fwd_kernel(const uint16_t * __restrict__ x, const uint16_t * __restrict__ 
 	  *yo = v;
 	}
 	if (act) {
-	  h4a a;
-#pragma unroll
-	  for (int i = 0; i < 4; i++) a[i] = silu_bf16(v[i]);
-	  *reinterpret_cast<h4a *>(act + o) = a;
+	  const float z[4] = {v[0], v[1], v[2], v[3]};
+	  uint16_t a[4];
+	  silu_bf16(z, a);
+	  *reinterpret_cast<h4a *>(act + o) = h4a{a[0], a[1], a[2], a[3]};
 	}
       }
     }

@@ -36,7 +36,12 @@ int grid_of(int64_t n) {
 
 // SiLU: a = z sigma(z)
 __global__ void silu_fwd_kernel(const float * __restrict__ z, uint16_t * __restrict__ a, int64_t n) {
-  GRID_STRIDE(i, n) a[i] = silu_bf16(z[i]);
+  GRID_STRIDE(i, n) {
+    const float v[1] = {z[i]};
+    uint16_t o[1];
+    silu_bf16(v, o);
+    a[i] = o[0];
+  }
 }
 
 // dz = da sigma(z) (1 + z (1 - sigma(z)))

@@ -191,6 +191,32 @@ def test_silu_backward_vector_path_is_the_scalar_one(n):
     assert np.allclose(out[0][0], da * sg * (1 + zz * (1 - sg)), rtol=1e-5, atol=1e-6)
 
 
+# The activation is the nearest BF16 value of z sigma(z) in FP32.  Four
+# roundings and the exponential's two ulp lie between that and the exact value
+# whatever |z| is, 6 u of the value at most (u = 2^-24); an exponent rounded
+# once would add |z| u.  Where the hardware's reciprocal is subnormal (below -87)
+# and past the exponential's range the result stays that of the division.
+def test_silu_is_rounded_from_full_precision():
+    lib = L.lib()
+    rng = np.random.default_rng(5)
+    n = 1 << 20
+    z = np.concatenate([-rng.uniform(0.1, 88.0, n), 8 * rng.standard_normal(n), -rng.uniform(80.0, 88.5, n // 16),
+                        rng.uniform(30.0, 300.0, n // 16), rng.standard_normal(n // 16) * 1e-20]).astype(np.float32)
+    d, a = dev(z, np.float32), L.DeviceArray(z.size, np.uint16)
+    assert lib.ldw_nn_silu_fwd(vp(d), vp(a), z.size) == 0
+    zz = z.astype(np.float64)
+    want = zz / (1 + np.exp(-zz))
+    half = np.exp2(np.floor(np.log2(np.abs(want))) - 8)
+    within(bf16_value(a.download()).astype(np.float64), want, half + 6 * EPS32 * np.abs(want), "silu")
+    z = np.array([0.0, -0.0, np.inf, np.nan, -np.inf, -89.0, -1e30, 1e30, 1e-40, -1e-40], np.float32)
+    d, a = dev(z, np.float32), L.DeviceArray(z.size, np.uint16)
+    assert lib.ldw_nn_silu_fwd(vp(d), vp(a), z.size) == 0
+    got = bf16_value(a.download())
+    with np.errstate(all="ignore"):
+        want = bf16_round(z / (1 + np.exp(-z)))
+    assert np.array_equal(got, want, equal_nan=True) and np.array_equal(np.signbit(got[:2]), [False, True])
+
+
 # 8 channels at a time or singly (odd counts of 8, off = 1: misaligned), against
 # float64 and each other
 @pytest.mark.parametrize("batch,shape,c", [(1, (2, 2, 2), 8), (2, (4, 6, 10), 40), (3, (2, 130, 66), 16)])
