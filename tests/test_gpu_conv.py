@@ -155,6 +155,33 @@ def test_conv_weight_gradient_tiles(cin, cout, batch, shape, accumulate):
     within(dw.download().astype(np.float64), want, 2 * (n + 1) * EPS32 * mag + 1e-30, "weight gradient")
 
 
+# Tiles that reach past the lattice hold zeros in one operand where the other
+# may hold values wrapped into it: an infinity of x or dy gives the sums that it
+# enters no NaN.  The corners' and an inner position, each in a channel of its
+# own; either operand shifted; ragged in y, in z, in both and not at all
+@pytest.mark.parametrize("cin,cout", [(16, 32), (48, 16)])
+@pytest.mark.parametrize("shape", [(2, 9, 16), (1, 8, 17), (3, 7, 18), (2, 8, 16), (2, 6, 3)])
+def test_conv_weight_gradient_infinities(cin, cout, shape):
+    lib = L.lib()
+    rng = np.random.default_rng(cin + shape[1])
+    n = int(np.prod(shape))
+    last = tuple(s - 1 for s in shape)
+    where = [(0, 0, 0), last, (0, last[1], 0), (0, 0, last[2]), (0, shape[1] // 2, shape[2] // 2)]
+    for k in range(2):
+        a = [bf16_round(rng.standard_normal(n * c)) for c in (cin, cout)]
+        for c, p in enumerate(where):
+            a[k].reshape(shape + (-1,))[p + (2 * c + 1,)] = np.inf
+        dx, dg = (dev(bf16_bits(v), np.uint16) for v in a)
+        dw = L.DeviceArray(27 * cout * cin, np.float32)
+        assert lib.ldw_conv3d_bwd_weight(vp(dx), vp(dg), vp(dw), 1, *shape, cin, cout, 0) == 0
+        with np.errstate(invalid="ignore"):
+            want = O.conv3_bwd_weight(a[0], a[1], shape, cin, cout, 1)
+        got = dw.download()
+        assert np.array_equal(np.isfinite(got), np.isfinite(want))
+        inf = np.isinf(want)
+        assert inf.any() and np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(got[inf], want[inf])
+
+
 # channel counts below, at and above what a block's 256 threads cover, 4 at a
 # time or singly, positions fewer and more than the blocks; off = 1 shifts the
 # array off 16-byte alignment
