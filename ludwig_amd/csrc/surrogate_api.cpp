@@ -158,6 +158,7 @@ extern "C" int ldw_nn_silu_bwd(const float * z, const float * da, float * dz, vo
 }
 
 extern "C" int ldw_nn_bias_grad(const float * dz, float * db, long long npos, int c, int accumulate) {
+  if (c < 1) LDW_FAIL("ldw_nn_bias_grad: %d channels", c);
   READY();
   void * work = nullptr;
   if (scratch_buffer(g_bias, (size_t) ldw::nn_bias_grad_workspace(npos, c)*sizeof(float), &work)) return -1;
