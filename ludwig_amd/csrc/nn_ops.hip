@@ -254,7 +254,7 @@ __global__ void pool2_fwd_kernel(const uint16_t * __restrict__ in, uint16_t * __
 }
 
 // the same, 8 channels (16 bytes) per thread and one z line of coarse positions
-// per block, for c a multiple of 8 and aligned arrays: bound by reading the fine
+// per block (or part of one), for c a multiple of 8 and aligned arrays: bound by reading the fine
 // array, where the kernel above divides 64-bit indices for each value and loads
 // 2 bytes at a time (the three levels of 8 x 64^3 at base 32, 235 MB read: about
 // 83 us above, 36 us here; the whole forward 1082 -> 1035 us).  Values are added
@@ -267,7 +267,7 @@ pool2_fwd8_kernel(const uint4 * __restrict__ in, uint4 * __restrict__ out, int64
     const int y = (int) (l % my), x = (int) ((l/my) % mx);
     const int64_t b = l/((int64_t) mx*my);
     const int64_t f0 = ((b*nx + 2*x)*ny + 2*y)*nz;
-    for (int i = threadIdx.x; i < mz*c8; i += 256) {
+    for (int i = blockIdx.y*256 + threadIdx.x; i < mz*c8; i += gridDim.y*256) {
       const int z = i/c8, k = i - z*c8;
       float s[8];
 #pragma unroll
@@ -678,8 +678,13 @@ hipError_t nn_pool2_fwd(const uint16_t * in, uint16_t * out, int batch, int nx, 
 			hipStream_t s) {
   if (c % 8 == 0 && (((uintptr_t) in | (uintptr_t) out) % 16) == 0) {
     const int64_t nline = (int64_t) batch*(nx/2)*(ny/2);
-    hipLaunchKernelGGL(pool2_fwd8_kernel, dim3((unsigned) (nline < 16384 ? (nline > 0 ? nline : 1) : 16384)), dim3(256),
-		       0, s, reinterpret_cast<const uint4 *>(in), reinterpret_cast<uint4 *>(out), nline, nx, ny, nz, c/8);
+    // few long lines are shared by several blocks each, up to 2048 in all (one
+    // line of 1000 coarse positions of 16 channels: 8.2 us in one block, 3.9 in 8)
+    const int64_t most = (nline > 0 && nline < 2048) ? 2048/nline : 1;
+    const int64_t split = ((int64_t) (nz/2)*(c/8) + 255)/256;
+    const dim3 grid((unsigned) (nline < 16384 ? (nline > 0 ? nline : 1) : 16384),
+		    (unsigned) (split < 1 ? 1 : (split < most ? split : most)));
+    hipLaunchKernelGGL(pool2_fwd8_kernel, grid, dim3(256), 0, s, reinterpret_cast<const uint4 *>(in), reinterpret_cast<uint4 *>(out), nline, nx, ny, nz, c/8);
     return hipGetLastError();
   }
   const int64_t n = (int64_t) batch*(nx/2)*(ny/2)*(nz/2)*c;

@@ -245,8 +245,9 @@ def test_silu_is_rounded_from_full_precision():
 
 
 # 8 channels at a time or singly (odd counts of 8, off = 1: misaligned), against
-# float64 and each other
-@pytest.mark.parametrize("batch,shape,c", [(1, (2, 2, 2), 8), (2, (4, 6, 10), 40), (3, (2, 130, 66), 16)])
+# float64 and each other; the last shapes' lines take several blocks each
+@pytest.mark.parametrize("batch,shape,c", [(1, (2, 2, 2), 8), (2, (4, 6, 10), 40), (3, (2, 130, 66), 16),
+                                           (1, (2, 2, 1030), 24), (2, (2, 4, 600), 16)])
 def test_pool_vector_path_is_the_scalar_one(batch, shape, c):
     lib = L.lib()
     rng = np.random.default_rng(c)
