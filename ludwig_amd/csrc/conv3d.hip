@@ -105,8 +105,9 @@ __device__ __forceinline__ int halo_at(int i, int n) {
 
 // 16 bytes per lane from global memory to LDS at byte offset `to` + 16 lane.
 // The compiler does not know that the load is in flight: wait_barrier waits.
+// The offset goes through M0, which the compiler sets.
 __device__ __forceinline__ void load_to_lds(const void * from, uint32_t to) {
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" :: "v"(from), "s"(to) : "memory");
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" :: "v"(from), "{m0}"(to) : "memory");
 }
 
 // all but this wave's last N memory operations and all its LDS reads done,
