@@ -47,17 +47,35 @@ binary_step_kernel(Geom g, FeParams fe, LbParams prm, int nbz, int nby, int nbx,
 					   u_prev, u_next, rho, g_in, g_out, fz0, fz1, fz2, csum);
 }
 
-// Blocks of this tile that the whole GPU holds at once (resident blocks per
-// CU from the occupancy of the order-1 kernel, times the CUs); cached.
-template <typename T, class S>
-int resident_slots() {
-  static int slots = 0;
+// The kernel for these parameters.  Advection order 4 is built for the 64 x 8
+// tile only (launch() picks it).
+template <typename T, class S, bool CONS, bool GMU>
+auto step_kernel(const FeParams & fe, const LbParams & prm) {
+  const bool gz = (prm.relax == 0);
+#define K_G(O, M) (gz ? &binary_step_kernel<T, S, O, M, true, CONS, GMU> \
+		   : &binary_step_kernel<T, S, O, M, false, CONS, GMU>)
+#define K_M(O) (fe.force_method == 0 ? K_G(O, 0) : K_G(O, 1))
+  if constexpr (S::TZ == 64) {
+    if (fe.order == 4) return K_M(4);
+  }
+  return fe.order == 1 ? K_M(1) : (fe.order == 2 ? K_M(2) : K_M(3));
+#undef K_M
+#undef K_G
+}
+
+// Blocks of that kernel that the whole GPU holds at once (resident blocks per
+// CU times the CUs); cached.  The kernels differ: FP32 with 32 x 8 tiles, 3 per
+// CU, but 2 with advection order 3.
+template <typename T, class S, bool CONS, bool GMU>
+int resident_slots(const FeParams & fe, const LbParams & prm) {
+  static int cache[5][2][2];
+  int & slots = cache[(fe.order >= 1 && fe.order <= 4) ? fe.order : 0][fe.force_method == 0][prm.relax == 0];
   if (slots == 0) {
     int per_cu = 0, dev = 0;
     hipDeviceProp_t prop;
+    const void * kernel = reinterpret_cast<const void *>(step_kernel<T, S, CONS, GMU>(fe, prm));
     if (hipGetDevice(&dev) != hipSuccess || hipGetDeviceProperties(&prop, dev) != hipSuccess
-	|| hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, binary_step_kernel<T, S, 1, 0, true, false, false>,
-							 S::NT, 0) != hipSuccess || per_cu < 1) {
+	|| hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, S::NT, 0) != hipSuccess || per_cu < 1) {
       (void) hipGetLastError();
       return 256;
     }
@@ -115,16 +133,17 @@ inline StepPlan rounds_plan(const Geom & g, int slots) {
 // and 1.25 M (FP32), and at 1.2 of padding (FP64 87x58x212, 1.21: 104 us with 64
 // x 8, 108 with 32 x 8; 82x173x150, 1.28: 237 and 209).
 template <typename T>
-StepPlan step_plan(const Geom & g) {
+StepPlan step_plan(const Geom & g, const FeParams & fe, const LbParams & prm) {
   static const int tzs[3] = {16, 32, 64};
-  const int slots[3] = {resident_slots<T, Shape<16, 8>>(), resident_slots<T, Shape<32, 8>>(),
-			resident_slots<T, Shape<64, 8>>()};
+  const int slots[3] = {resident_slots<T, Shape<16, 8>, false, false>(fe, prm),
+			resident_slots<T, Shape<32, 8>, false, false>(fe, prm),
+			resident_slots<T, Shape<64, 8>, false, false>(fe, prm)};
   // a plane of the narrower tiles costs slightly more or less than its share
   static const double weight64[3] = {1.00, 1.02, 1.10}, weight32[3] = {1.05, 1.00, 1.10};
   const double * weight = (sizeof(T) == 8) ? weight64 : weight32;
   const int64_t small = (sizeof(T) == 8) ? 800000 : 1250000;
   const int forced = tune_step_tile();
-  if (g.nsite <= small || forced) {
+  if (g.nsite <= small) {
     StepPlan best = {0, 0, 1};
     double best_cost = 0.0;
     for (int k = 0; k < 3; k++) {
@@ -135,14 +154,14 @@ StepPlan step_plan(const Geom & g) {
       const double cost = (double) (xc + 2)*weight[k];
       if (best.tz == 0 || cost < best_cost) { best = {tzs[k], (int) ceil_div(g.nx, xc), 1}; best_cost = cost; }
     }
-    if (best.tz && g.nsite <= small) return best;
+    if (best.tz) return best;
   }
   if (forced == 64 || (!forced && ceil_div(g.nz, 64)*64*5 <= (int64_t) g.nz*6))
     return rounds_plan(g, slots[2]);
   return {forced ? forced : 32, (int) ceil_div(g.nx, 3), 1};
 }
 
-template <typename T, class S, bool CONS, bool GMU = false>
+template <typename T, class S, bool CONS, bool GMU>
 void launch_shape(const Geom & g, const FeParams & fe, const LbParams & prm, const T * phi,
 		  T * phi_out, const T * u_prev, T * u_next, T * rho, const T * g_in,
 		  T * g_out, const double fzero[3], T * csum, const StepPlan & plan, hipStream_t st) {
@@ -159,22 +178,8 @@ void launch_shape(const Geom & g, const FeParams & fe, const LbParams & prm, con
   const int ntile = bz*by*bx;
   dim3 grid(((ntile + NXCD - 1)/NXCD)*NXCD), block(S::TZ, S::TY, 1);
   const T f0 = T(fzero[0]), f1 = T(fzero[1]), f2 = T(fzero[2]);
-  const bool gz = (prm.relax == 0);
-#define L_(O, M, G) hipLaunchKernelGGL((binary_step_kernel<T, S, O, M, G, CONS, GMU>), grid, block, 0, st, \
-				       g, fe, prm, bz, by, bx, tune_remap_step(plan.remap), phi, phi_out, u_prev, u_next, rho, \
-				       g_in, g_out, f0, f1, f2, csum)
-#define L_G(O, M) do { if (gz) L_(O, M, true); else L_(O, M, false); } while (0)
-#define L_M(O) do { if (fe.force_method == 0) L_G(O, 0); else L_G(O, 1); } while (0)
-  if (fe.order == 4) {
-    // advection order 4 is built for the 64 x 8 tile only (launch() picks it)
-    if constexpr (S::TZ == 64 && S::TY == 8) L_M(4);
-  }
-  else if (fe.order == 1) L_M(1);
-  else if (fe.order == 2) L_M(2);
-  else L_M(3);
-#undef L_M
-#undef L_G
-#undef L_
+  hipLaunchKernelGGL((step_kernel<T, S, CONS, GMU>(fe, prm)), grid, block, 0, st, g, fe, prm, bz, by, bx,
+		     tune_remap_step(plan.remap), phi, phi_out, u_prev, u_next, rho, g_in, g_out, f0, f1, f2, csum);
 }
 
 // The tile changes only which block computes a site, not the arithmetic.
@@ -187,20 +192,18 @@ void launch(const Geom & g, const FeParams & fe, const LbParams & prm, const T *
 	    T * phi_out, const T * u_prev, T * u_next, T * rho, const T * g_in,
 	    T * g_out, const double fzero[3], T * csum, hipStream_t st) {
   using S64 = Shape<64, 8>;
+#define S64_(CONS, GMU) launch_shape<T, S64, CONS, GMU>(g, fe, prm, phi, phi_out, u_prev, u_next, rho, g_in, g_out, fzero, \
+						       csum, rounds_plan(g, resident_slots<T, S64, CONS, GMU>(fe, prm)), st)
   if (fe.gmu_on || csum || fe.order == 4) {
-    const StepPlan n = rounds_plan(g, resident_slots<T, S64>());
-    if (fe.gmu_on && csum) launch_shape<T, S64, true, true>(g, fe, prm, phi, phi_out, u_prev, u_next, rho, g_in,
-							    g_out, fzero, csum, n, st);
-    else if (fe.gmu_on) launch_shape<T, S64, false, true>(g, fe, prm, phi, phi_out, u_prev, u_next, rho, g_in,
-							  g_out, fzero, nullptr, n, st);
-    else if (csum) launch_shape<T, S64, true>(g, fe, prm, phi, phi_out, u_prev, u_next, rho, g_in, g_out, fzero,
-					      csum, n, st);
-    else launch_shape<T, S64, false>(g, fe, prm, phi, phi_out, u_prev, u_next, rho, g_in, g_out, fzero,
-				     nullptr, n, st);
+    if (fe.gmu_on && csum) S64_(true, true);
+    else if (fe.gmu_on) S64_(false, true);
+    else if (csum) S64_(true, false);
+    else S64_(false, false);
     return;
   }
-  const StepPlan p = step_plan<T>(g);
-#define TILE_(TZ) launch_shape<T, Shape<TZ, 8>, false>(g, fe, prm, phi, phi_out, u_prev, u_next, rho, g_in, g_out, \
+#undef S64_
+  const StepPlan p = step_plan<T>(g, fe, prm);
+#define TILE_(TZ) launch_shape<T, Shape<TZ, 8>, false, false>(g, fe, prm, phi, phi_out, u_prev, u_next, rho, g_in, g_out, \
 						       fzero, nullptr, p, st)
   if (p.tz == 16) TILE_(16);
   else if (p.tz == 32) TILE_(32);
