@@ -1,7 +1,7 @@
 // fe_ch_fused.hip -- K23: thermodynamic force and Cahn-Hilliard update of
 // the symmetric free energy in one pass over phi.
 //
-// One block owns a TY x TZ (8 x 16) tile of (y, z) columns and marches along x.  LDS
+// One block owns a TY x TZ tile of (y, z) columns and marches along x.  LDS
 // holds a ring of 5 phi planes with a halo of 2 in y and z, and a ring of 3
 // planes of Q = (d_x phi, d_y phi, d_z phi, p0, mu) with a halo of 1, so
 // every phi value is fetched from memory about once and every stencil
@@ -21,6 +21,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include "chunk_plan.h"
 #include "kernels.h"
 #include "fe_tile.h"
 
@@ -101,44 +102,25 @@ force_ch_kernel(Geom g, FeParams fe, int nbz, int nby, int nbx, int remap, const
 }
 
 template <typename T, class S>
-void launch_shape(const Geom & g, const FeParams & fe, const T * phi, const T * u, T * force,
-		  T * phi_out, T * csum, int force_mode, const double fzero[3], int bx, hipStream_t st) {
-  const int bz = (g.nz + S::TZ - 1)/S::TZ;
-  const int by = (g.ny + S::TY - 1)/S::TY;
-  const int ntile = bz*by*bx;
-  dim3 grid(((ntile + NXCD - 1)/NXCD)*NXCD), block(S::TZ, S::TY, 1);
-  const T f0 = T(fzero[0]), f1 = T(fzero[1]), f2 = T(fzero[2]);
-#define L_(O, M, U) hipLaunchKernelGGL((force_ch_kernel<T, S, O, M, U>), grid, block, 0, st, \
-				       g, fe, bz, by, bx, tune_remap(), phi, u, force, phi_out, csum, force_mode, \
-				       f0, f1, f2)
-#define L_U(O, M) do { if (u) L_(O, M, true); else L_(O, M, false); } while (0)
-#define L_M(O) do { if (fe.force_method == 0) L_U(O, 0); else L_U(O, 1); } while (0)
-  if (fe.order == 1) L_M(1);
-  else if (fe.order == 2) L_M(2);
-  else if (fe.order == 3) L_M(3);
-  else L_M(4);
-#undef L_M
-#undef L_U
-#undef L_
+auto force_ch_of(const FeParams & fe, bool have_u) {
+#define K_U(O, M) (have_u ? &force_ch_kernel<T, S, O, M, true> : &force_ch_kernel<T, S, O, M, false>)
+#define K_M(O) (fe.force_method == 0 ? K_U(O, 0) : K_U(O, 1))
+  return fe.order == 1 ? K_M(1) : (fe.order == 2 ? K_M(2) : (fe.order == 3 ? K_M(3) : K_M(4)));
+#undef K_M
+#undef K_U
 }
 
-// Tile and chunks: 16 x 8 tiles in one round of as many blocks as the GPU
-// holds (5 per CU in FP64).  The pass reads and writes little, so it is bound
-// by the length of a block (prologue and planes in a row), not by memory.
-// us at 100x84x76 / 128^3 / 144^3 FP64: 26 / 57 / 79, against 47 / 73 / 149 for 64 x
-// 4 tiles in 2048 blocks (the second round of which repeats the prologue) and
-// 33 / 65 / 84 for 32 x 8 tiles at their best; FP32 21 / 40 / 54 against 27 / 45 / 88.
-using S16 = Shape<16, 8>;
-
-template <typename T>
-int resident_slots() {
-  static int slots = 0;
+// Blocks of that kernel that the whole GPU holds at once; cached.
+template <typename T, class S>
+int resident_slots(const FeParams & fe, bool have_u) {
+  static int cache[5][2][2];
+  int & slots = cache[(fe.order >= 1 && fe.order <= 4) ? fe.order : 0][fe.force_method == 0][have_u];
   if (slots == 0) {
     int per_cu = 0, dev = 0;
     hipDeviceProp_t prop;
+    const void * kernel = reinterpret_cast<const void *>(force_ch_of<T, S>(fe, have_u));
     if (hipGetDevice(&dev) != hipSuccess || hipGetDeviceProperties(&prop, dev) != hipSuccess
-	|| hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, force_ch_kernel<T, S16, 1, 0, true>, S16::NT, 0)
-	   != hipSuccess || per_cu < 1) {
+	|| hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, S::NT, 0) != hipSuccess || per_cu < 1) {
       (void) hipGetLastError();
       return 1024;
     }
@@ -147,15 +129,42 @@ int resident_slots() {
   return slots;
 }
 
+template <class S>
+int64_t columns(const Geom & g) {
+  return (int64_t) ((g.nz + S::TZ - 1)/S::TZ)*((g.ny + S::TY - 1)/S::TY);
+}
+
+template <typename T, class S>
+void launch_shape(const Geom & g, const FeParams & fe, const T * phi, const T * u, T * force,
+		  T * phi_out, T * csum, int force_mode, const double fzero[3], hipStream_t st) {
+  const int bz = (g.nz + S::TZ - 1)/S::TZ;
+  const int by = (g.ny + S::TY - 1)/S::TY;
+  const int bx = chunk_count(g.nx, columns<S>(g), resident_slots<T, S>(fe, u != nullptr));
+  const int ntile = bz*by*bx;
+  dim3 grid(((ntile + NXCD - 1)/NXCD)*NXCD), block(S::TZ, S::TY, 1);
+  const T f0 = T(fzero[0]), f1 = T(fzero[1]), f2 = T(fzero[2]);
+  hipLaunchKernelGGL((force_ch_of<T, S>(fe, u != nullptr)), grid, block, 0, st, g, fe, bz, by, bx, tune_remap(), phi, u,
+		     force, phi_out, csum, force_mode, f0, f1, f2);
+}
+
+// Tile: 16 x 8 in FP64, 32 x 8 in FP32, whose 16-wide rows fill half a cache
+// line, except where every plane of every 16 x 8 column runs at once.
+// Measured over 16 lattices of 24^3 to 256^3, 300x160x160 to 20x1000x600, with
+// tiles of 16 x 8, 32 x 4, 32 x 8, 64 x 4 and 64 x 8 and 256 to 4096 blocks:
+// the chunks of chunk_count are the best ones of their tile but for flat
+// lattices (at most 8 % off).  us of FP64 128x200x400 / 256x200x200 / 256^3:
+// 252 / 263 / 394, with 64 x 4 tiles at their best 328 / 345 / 424, with
+// 64 x 4 in 2048 blocks 338 / 387 / 442, with 16 x 8 in a single round 331 /
+// 263 / 396.  FP32 64x288x288 / 256^3 / 40x640x300: 69 / 210 / 121, with 64 x 4
+// in 2048 blocks 89 / 224 / 120, with 16 x 8 86 / 281 / 150.
 template <typename T>
 void launch(const Geom & g, const FeParams & fe, const T * phi, const T * u, T * force,
 	    T * phi_out, T * csum, int force_mode, const double fzero[3], hipStream_t st) {
-  const int64_t ncol = (int64_t) ((g.nz + 15)/16)*((g.ny + 7)/8);
-  // more columns than slots: chunks of 16 planes
-  int64_t bx = resident_slots<T>()/ncol;
-  if (bx < 1) bx = (g.nx + 15)/16;
-  if (bx > g.nx) bx = g.nx;
-  launch_shape<T, S16>(g, fe, phi, u, force, phi_out, csum, force_mode, fzero, (int) bx, st);
+  using S16 = Shape<16, 8>;
+  if (sizeof(T) == 8 || columns<S16>(g)*g.nx <= resident_slots<T, S16>(fe, u != nullptr))
+    launch_shape<T, S16>(g, fe, phi, u, force, phi_out, csum, force_mode, fzero, st);
+  else if constexpr (sizeof(T) == 4)
+    launch_shape<T, Shape<32, 8>>(g, fe, phi, u, force, phi_out, csum, force_mode, fzero, st);
 }
 
 }  // namespace

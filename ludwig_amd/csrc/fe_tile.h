@@ -22,7 +22,7 @@ namespace tile {
 // Tile shape: TZ x TY sites of a plane, one thread per site (block
 // dimensions (TZ, TY)).  The single-lattice step chooses 16 x 8, 32 x 8 or
 // 64 x 8 by precision and lattice (step_plan); the staged force/Cahn-Hilliard
-// kernel uses 16 x 8; the replica ensemble chooses among several shapes at
+// kernel uses 16 x 8 and 32 x 8; the replica ensemble chooses among several shapes at
 // run time (ensemble.hip).
 template <int TZ_, int TY_>
 struct Shape {

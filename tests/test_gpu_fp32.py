@@ -96,3 +96,31 @@ def test_fp32_256_against_fp64():
     (r0, p0), (r1, p1) = out[32][3], out[32][4]
     assert abs(r1 - r0) / r0 < 1e-9
     assert abs(p1 - p0) / n ** 3 < 1e-8
+
+
+# The staged force and Cahn-Hilliard pass takes 16 x 8 tiles where all of its
+# planes run at once, 32 x 8 tiles in chunks elsewhere: the same bits.  The
+# small lattices take the first, their repetitions (3600 and 8000 column planes for at
+# most 2560 resident blocks) the second.
+@pytest.mark.parametrize("order", [1, 3])
+@pytest.mark.parametrize("small,reps", [((8, 40, 50), (3, 3, 3)), ((5, 33, 47), (2, 9, 7))])
+def test_fp32_staged_tiles_agree(small, reps, order):
+    shapes = (small, tuple(a * b for a, b in zip(small, reps)))
+    phi = 0.5 * np.random.default_rng(small[1]).standard_normal(small).astype(np.float32)
+    out = []
+    for shape in shapes:
+        b = L.BinaryFluid(shape, tau=1.0, mobility=0.25, order=order, precision=32)
+        b.init_rest()
+        b.set_phi(np.tile(phi, tuple(a // c for a, c in zip(shape, small))).ravel())
+        for _ in range(2):
+            b.f_zero()
+            b.force_stage()
+            b.cahn_hilliard_stage()
+            b.u_zero()
+            b.collide(b.fe)
+            b.propagate()
+        rho, u, force = b.hydro_fields()
+        out.append([a.reshape((-1,) + shape) for a in (b.phi_field(), rho, u, force)])
+        b.close()
+    for name, a, c in zip(("phi", "rho", "u", "force"), *out):
+        assert np.array_equal(np.tile(a, (1,) + reps), c), name
