@@ -21,6 +21,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "conv_plan.h"
 #include "kernels.h"
 #include "silu.h"
 
@@ -117,7 +118,10 @@ __device__ __forceinline__ void wait_barrier() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(N) : "memory");
 }
 
-template <int NT, int TY, int ZT>
+// DMA: x and w are 16-byte aligned, as the loads to LDS need it.  Otherwise the
+// same loads go through registers: requested at the same places, written to
+// LDS at the unit's end (weights) and the next unit's (halo).
+template <int NT, int TY, int ZT, bool DMA>
 __global__ void __launch_bounds__(256, 2)
 conv3_fwd_kernel(const uint16_t * __restrict__ x, const uint16_t * __restrict__ w,
 		 const float * __restrict__ bias, float * __restrict__ y, uint16_t * __restrict__ act,
@@ -161,13 +165,21 @@ conv3_fwd_kernel(const uint16_t * __restrict__ x, const uint16_t * __restrict__ 
     }
   };
   // loads [i0, i1) of slice c0 of the sample at tp into halo buffer hb
+  u4 rh[C::HW], rw[WW];                       // (not DMA) in flight
+  auto halo_row = [&](int i, int hb) { return 2*NW + 64*(hb*C::HL + min(wave + 4*i, C::HL - 1)); };
   auto fetch_halo = [&](int i0, int i1, int64_t tp, int c0, int hb) {
 #pragma unroll
     for (int i = 0; i < C::HW; i++) {
       if (i < i0 || i >= i1) continue;
-      load_to_lds(x + (tp + hs[i])*cin + (c0 + 8*(hc[i] >> 24)),
-		  base + 16*(2*NW + 64*(hb*C::HL + min(wave + 4*i, C::HL - 1))));
+      const uint16_t * from = x + (tp + hs[i])*cin + (c0 + 8*(hc[i] >> 24));
+      if constexpr (DMA) load_to_lds(from, base + 16*halo_row(i, hb));
+      else rh[i] = *reinterpret_cast<const u4a *>(from);
     }
+  };
+  auto put_halo = [&](int i0, int i1, int hb) {
+#pragma unroll
+    for (int i = 0; i < C::HW; i++)
+      if (i >= i0 && i < i1) lds[halo_row(i, hb) + lane] = rh[i];
   };
 
   // This lane's weight vectors: row dy*16*NT + n, part; parts 2, 3 belong to
@@ -181,13 +193,20 @@ conv3_fwd_kernel(const uint16_t * __restrict__ x, const uint16_t * __restrict__ 
     const int n = min(n0 + row % (16*NT), cout - 1);
     wo[k] = ((3*(row/(16*NT))*cout + n)*cin + 8*(part & 1))*2 + (part >> 1);
   }
+  auto w_row = [&](int k, int buf) { return buf*NW + 64*min(wave + 4*k, WL - 1); };
   auto fetch_w = [&](int u, int c0, int buf) {
     // second column: dz + 1 (units 0-2), dx + 1 (unit 3), none (unit 4)
     const int col = (u < 3) ? 9*u : (u == 3 ? 2 : 20), step = (u < 3) ? 1 : (u == 3 ? 9 : 0);
 #pragma unroll
-    for (int k = 0; k < WW; k++)
-      load_to_lds(w + ((int64_t) col*tap + c0) + ((wo[k] >> 1) + (wo[k] & 1)*(step*tap)),
-		  base + 16*(buf*NW + 64*min(wave + 4*k, WL - 1)));
+    for (int k = 0; k < WW; k++) {
+      const uint16_t * from = w + ((int64_t) col*tap + c0) + ((wo[k] >> 1) + (wo[k] & 1)*(step*tap));
+      if constexpr (DMA) load_to_lds(from, base + 16*w_row(k, buf));
+      else rw[k] = *reinterpret_cast<const u4a *>(from);
+    }
+  };
+  auto put_w = [&](int buf) {
+#pragma unroll
+    for (int k = 0; k < WW; k++) lds[w_row(k, buf) + lane] = rw[k];
   };
 
   f4 acc[TY][NT];
@@ -293,6 +312,7 @@ conv3_fwd_kernel(const uint16_t * __restrict__ x, const uint16_t * __restrict__ 
   sites(x0, y0, z0);
   fetch_w(0, 0, 0);
   fetch_halo(0, C::HW, p0, 0, 0);
+  if constexpr (!DMA) { put_w(0); put_halo(0, C::HW, 0); }
   wait_barrier<0>();
   int buf = 0, hb = 0, c0 = 0;
 #pragma unroll 1
@@ -317,6 +337,10 @@ conv3_fwd_kernel(const uint16_t * __restrict__ x, const uint16_t * __restrict__ 
       if (u < 3) unit32(buf, hb, u, hi);
       else if (u == 3) unit32(buf, hb, hi, 2);
       else unit16(buf, hb);
+      if constexpr (!DMA) {
+	put_w(buf ^ 1);
+	if (u > 0) put_halo((u - 1)*C::HU, u*C::HU, hb ^ 1);
+      }
       // wait for the weights; this unit's halo loads may go on
       if (u == 0) wait_barrier<C::in_unit(0)>();
       else if (u == 1) wait_barrier<C::in_unit(1)>();
@@ -614,39 +638,7 @@ int grid_for(int64_t n) {
   return (int) (g < 8192 ? (g > 0 ? g : 1) : 8192);
 }
 
-constexpr int CONV_BLOCKS = 512;              // two per CU
-
-struct ConvShape { int nt, ty, zt; };
-
-// Output channels per block (16 nt), rows per wave and depth of the tile.
-//
-// A wave wants 8 rows (a halo row is then read 1.25 times instead of 1.5) as
-// long as that makes enough blocks, with up to 32 channels: 8 rows and 48 do
-// not fit LDS twice.  80 -> 32 channels on 8 x 64^3: 357 us with (2, 8), 396
-// with (2, 4), 459 with (1, 8).  Wider layers take 3 or 4 blocks of 16,
-// whichever pads less (32 -> 48 on 8 x 32^3: 32 us with nt = 3, 37 with 2, 36
-// with 4), and fewer where the grid would not give each CU two blocks (64 ->
-// 64 on 8 x 16^3: 22 us with nt = 4, 17 with 2 or 1).
-ConvShape conv_shape(int batch, int nx, int ny, int nz, int nb16) {
-  ConvShape c;
-  c.zt = (nz > 8) ? 16 : 8;
-  const int cx = 4*16/c.zt;
-  auto tiles = [&](int ty) {
-    return (int64_t) batch*((nx + cx - 1)/cx)*((ny + ty - 1)/ty)*((nz + c.zt - 1)/c.zt);
-  };
-  c.ty = 4;
-  if (nb16 <= 2) {
-    c.nt = nb16;
-    if (tiles(8) >= CONV_BLOCKS) c.ty = 8;
-  }
-  else {
-    c.nt = ((nb16 + 3)/4*4 <= (nb16 + 2)/3*3) ? 4 : 3;
-  }
-  while (c.nt > 1 && tiles(c.ty)*((nb16 + c.nt - 1)/c.nt) < CONV_BLOCKS) c.nt--;
-  return c;
-}
-
-template <int NT, int TY, int ZT>
+template <int NT, int TY, int ZT, bool DMA>
 void launch_conv(const uint16_t * x, const uint16_t * w, const float * bias, float * y, uint16_t * act,
 		 int batch, int nx, int ny, int nz, int cin, int cout, int accumulate, hipStream_t s) {
   constexpr int X = ConvTile<TY, ZT>::X;
@@ -656,7 +648,7 @@ void launch_conv(const uint16_t * x, const uint16_t * w, const float * bias, flo
   if (nblk < 1) nblk = 1;
   if (nblk >= NXCD) nblk -= nblk % NXCD;
   if (nblk > ntile) nblk = ntile;
-  hipLaunchKernelGGL((conv3_fwd_kernel<NT, TY, ZT>), dim3(nblk, nb), dim3(256), 0, s, x, w, bias, y, act, nx, ny, nz,
+  hipLaunchKernelGGL((conv3_fwd_kernel<NT, TY, ZT, DMA>), dim3(nblk, nb), dim3(256), 0, s, x, w, bias, y, act, nx, ny, nz,
 		     cin, cout, accumulate, ntx, nty, ntz, ntile);
 }
 
@@ -666,22 +658,26 @@ hipError_t launch_conv3_fwd(const uint16_t * x, const uint16_t * w, const float 
 			    uint16_t * act, int batch, int nx, int ny, int nz, int cin, int cout,
 			    int accumulate, hipStream_t s) {
   const int nb16 = cout/16;
-  const ConvShape c = conv_shape(batch, nx, ny, nz, nb16);
-#define CONV_(NT, TY, ZT) launch_conv<NT, TY, ZT>(x, w, bias, y, act, batch, nx, ny, nz, cin, cout, accumulate, s)
-#define CONV_NT(NT, TY) do { if (c.zt == 16) CONV_(NT, TY, 16); else CONV_(NT, TY, 8); } while (0)
+  const bool dma = (((uintptr_t) x | (uintptr_t) w) % 16 == 0);
+  const ConvShape c = conv_shape(batch, nx, ny, nz, nb16, dma);
+#define CONV_(NT, TY, ZT, DMA) \
+  launch_conv<NT, TY, ZT, DMA>(x, w, bias, y, act, batch, nx, ny, nz, cin, cout, accumulate, s)
+#define CONV_Z(NT, TY, DMA) do { if (c.zt == 16) CONV_(NT, TY, 16, DMA); else CONV_(NT, TY, 8, DMA); } while (0)
+#define CONV_4(NT) do { if (dma) CONV_Z(NT, 4, true); else CONV_Z(NT, 4, false); } while (0)
   if (c.ty == 8) {
-    if (c.nt == 2) CONV_NT(2, 8);
-    else CONV_NT(1, 8);
+    if (c.nt == 2) CONV_Z(2, 8, true);
+    else CONV_Z(1, 8, true);
   }
   else {
     switch (c.nt) {
-    case 4: CONV_NT(4, 4); break;
-    case 3: CONV_NT(3, 4); break;
-    case 2: CONV_NT(2, 4); break;
-    default: CONV_NT(1, 4); break;
+    case 4: CONV_4(4); break;
+    case 3: CONV_4(3); break;
+    case 2: CONV_4(2); break;
+    default: CONV_4(1); break;
     }
   }
-#undef CONV_NT
+#undef CONV_4
+#undef CONV_Z
 #undef CONV_
   return hipGetLastError();
 }

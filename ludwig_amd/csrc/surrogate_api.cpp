@@ -22,7 +22,7 @@ struct Scratch {
   size_t bytes = 0;
 };
 
-Scratch g_wgrad, g_bias, g_err, g_sum, g_sumsq, g_restore, g_align_x, g_align_w;
+Scratch g_wgrad, g_bias, g_err, g_sum, g_sumsq, g_restore;
 
 int scratch_buffer(Scratch & s, size_t bytes, void ** out) {
   if (s.bytes < bytes) {
@@ -42,26 +42,6 @@ int check_conv(int batch, int nx, int ny, int nz, int cin, int cout) {
   if (batch < 1 || nx < 1 || ny < 1 || nz < 1) LDW_FAIL("conv3d: bad sizes %d x %d x %d x %d", batch, nx, ny, nz);
   if (cin < 16 || cout < 16 || cin % 16 || cout % 16)
     LDW_FAIL("conv3d: channel counts must be multiples of 16 (cin %d, cout %d)", cin, cout);
-  return 0;
-}
-
-// *p itself where it is 16-byte aligned, as the convolution's loads to LDS
-// need it, else a copy in scratch s
-int align16(const void ** p, size_t bytes, Scratch & s) {
-  if ((uintptr_t) *p % 16 == 0) return 0;
-  void * q = nullptr;
-  if (scratch_buffer(s, bytes, &q)) return -1;
-  LDW_HIP_CHECK(hipMemcpyAsync(q, *p, bytes, hipMemcpyDeviceToDevice, ldw::api::stream()));
-  *p = q;
-  return 0;
-}
-
-int conv_fwd(const void * x, const void * w, const float * bias, float * y, void * act, int batch, int nx,
-	     int ny, int nz, int cin, int cout, int accumulate) {
-  if (align16(&x, (size_t) batch*nx*ny*nz*cin*2, g_align_x)) return -1;
-  if (align16(&w, (size_t) 27*cin*cout*2, g_align_w)) return -1;
-  LDW_HIP_CHECK(ldw::launch_conv3_fwd((const uint16_t *) x, (const uint16_t *) w, bias, y, (uint16_t *) act, batch,
-				      nx, ny, nz, cin, cout, accumulate, ldw::api::stream()));
   return 0;
 }
 
@@ -105,7 +85,9 @@ extern "C" int ldw_conv3d_fwd(const void * x, const void * w, const float * bias
   READY();
   if (check_conv(batch, nx, ny, nz, cin, cout)) return -1;
   if (y == nullptr) LDW_FAIL("ldw_conv3d_fwd: null output");
-  return conv_fwd(x, w, bias, y, nullptr, batch, nx, ny, nz, cin, cout, accumulate);
+  KCHECK(ldw::launch_conv3_fwd((const uint16_t *) x, (const uint16_t *) w, bias, y, nullptr, batch, nx,
+			       ny, nz, cin, cout, accumulate, ldw::api::stream()));
+  return 0;
 }
 
 extern "C" int ldw_conv3d_fwd_silu(const void * x, const void * w, const float * bias, float * z, void * a,
@@ -113,7 +95,9 @@ extern "C" int ldw_conv3d_fwd_silu(const void * x, const void * w, const float *
   READY();
   if (check_conv(batch, nx, ny, nz, cin, cout)) return -1;
   if (a == nullptr) LDW_FAIL("ldw_conv3d_fwd_silu: null activation output");
-  return conv_fwd(x, w, bias, z, a, batch, nx, ny, nz, cin, cout, 0);
+  KCHECK(ldw::launch_conv3_fwd((const uint16_t *) x, (const uint16_t *) w, bias, z, (uint16_t *) a, batch,
+			       nx, ny, nz, cin, cout, 0, ldw::api::stream()));
+  return 0;
 }
 
 extern "C" int ldw_conv3d_bwd_data(const void * dy, const void * wd, float * dx, int batch, int nx,
@@ -122,7 +106,9 @@ extern "C" int ldw_conv3d_bwd_data(const void * dy, const void * wd, float * dx,
   if (check_conv(batch, nx, ny, nz, cin, cout)) return -1;
   // dx (cin channels) = convolution of dy (cout channels) with the flipped,
   // transposed weights
-  return conv_fwd(dy, wd, nullptr, dx, nullptr, batch, nx, ny, nz, cout, cin, accumulate);
+  KCHECK(ldw::launch_conv3_fwd((const uint16_t *) dy, (const uint16_t *) wd, nullptr, dx, nullptr, batch,
+			       nx, ny, nz, cout, cin, accumulate, ldw::api::stream()));
+  return 0;
 }
 
 extern "C" int ldw_conv3d_bwd_weight(const void * x, const void * dy, float * dw, int batch, int nx,

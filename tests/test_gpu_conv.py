@@ -45,8 +45,7 @@ def within(got, want, bound, what):
                     f"(bound {bound[i]:.3e})")
 
 
-# lattices below 4 x 4 x 16 take the fragment-direct kernel, the rest the
-# LDS-tiled one (ragged tiles and 16-channel chunks included)
+# lattices that fill no tile, one and several, slices that end on 16 channels
 @pytest.mark.parametrize("cin,cout,batch,shape", [
     (16, 16, 1, SHAPE), (32, 48, 2, SHAPE), (48, 64, 1, SHAPE), (16, 96, 2, SHAPE),
     (32, 160, 1, SHAPE), (160, 32, 1, SHAPE),
@@ -101,12 +100,10 @@ def test_conv_fwd_bwd_against_oracle(cin, cout, batch, shape):
     within(y.download().astype(np.float64), 2 * yo, 4 * 27 * cin * EPS32 * ya + 1e-30, "forward x2")
 
 
-# the forward tiles: 4 or 8 rows of 16 z or 2 x 8 z per wave, 4 (or 8) x deep;
-# lattices of one site, one below, at and one above a tile's edges, slices
-# that end on 16 channels, output blocks that pad (5, 7), more tiles than
-# blocks (the last shapes: 8-row tiles and 16-channel outputs), in an order of
-# tiles that does and does not divide by the 8 XCDs; off shifts x and w off
-# 16-byte alignment
+# the forward kernels at the edges of their tiles: lattices of one site, one
+# below, at and one above a tile, slices that end on 16 channels, output blocks
+# that pad (5, 7), more tiles than blocks; off shifts x and w off 16-byte
+# alignment
 @pytest.mark.parametrize("cin,cout,batch,shape,off", [
     (16, 16, 1, (1, 1, 1), 0), (16, 32, 1, (3, 3, 7), 1), (32, 16, 1, (4, 4, 8), 0), (48, 80, 1, (9, 5, 8), 0),
     (16, 48, 2, (5, 5, 9), 1), (32, 112, 1, (4, 3, 17), 0), (64, 64, 1, (2, 9, 16), 0), (16, 128, 1, (1, 4, 31), 0),
@@ -128,6 +125,27 @@ def test_conv_forward_tiles(cin, cout, batch, shape, off):
         assert lib.ldw_conv3d_fwd(at(dx, 8 * off), at(dw, 8 * off), vp(db), vp(dy), batch, *shape, cin, cout, acc) == 0
         within(dy.download().astype(np.float64), want + acc * before,
                2 * (27 * cin + 2) * EPS32 * (mag + acc * np.abs(before)) + 1e-30, f"forward accumulate={acc}")
+
+
+# operands off 16-byte alignment are read where they are: no copy is kept
+def test_conv_misaligned_operands_take_no_memory():
+    lib = L.lib()
+    hip = ctypes.CDLL("libamdhip64.so.7")
+
+    def free():
+        assert lib.ldw_device_synchronize() == 0
+        a, b = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(a), ctypes.byref(b)) == 0
+        return a.value
+
+    batch, shape, cin, cout = 4, (64, 64, 64), 48, 16
+    n = batch * int(np.prod(shape))
+    zeros = lambda k: dev(np.zeros(k, np.uint16), np.uint16)
+    x, w, y = zeros(n * cin + 4), zeros(27 * cin * cout + 4), L.DeviceArray(n * cout, np.float32)
+    before = free()
+    assert lib.ldw_conv3d_fwd(at(x, 8), at(w, 8), None, vp(y), batch, *shape, cin, cout, 0) == 0
+    assert before - free() < n * cin
+    assert not y.download().any()
 
 
 # the weight gradient's tiles are 8 x 16 (y, z) columns marched along x: one
