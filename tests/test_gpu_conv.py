@@ -9,6 +9,8 @@ the weight gradient), with sum |a b| from the checker applied to |a|, |b|.
 """
 
 import ctypes
+import os
+import subprocess
 
 import numpy as np
 import pytest
@@ -125,6 +127,79 @@ def test_conv_forward_tiles(cin, cout, batch, shape, off):
         assert lib.ldw_conv3d_fwd(at(dx, 8 * off), at(dw, 8 * off), vp(db), vp(dy), batch, *shape, cin, cout, acc) == 0
         within(dy.download().astype(np.float64), want + acc * before,
                2 * (27 * cin + 2) * EPS32 * (mag + acc * np.abs(before)) + 1e-30, f"forward accumulate={acc}")
+
+
+@pytest.fixture(scope="module")
+def conv_shape(tmp_path_factory):
+    """The library's own choice of kernel (csrc/conv_plan.h): (nt, ty, zt)."""
+    d = tmp_path_factory.mktemp("plan")
+    (d / "plan.cpp").write_text("""
+#include "conv_plan.h"
+extern "C" void shape(int b, int nx, int ny, int nz, int cout, int dma, int * o) {
+  const ldw::ConvShape c = ldw::conv_shape(b, nx, ny, nz, cout/16, dma != 0);
+  o[0] = c.nt; o[1] = c.ty; o[2] = c.zt;
+}
+""")
+    csrc = os.path.join(os.path.dirname(L.__file__), "csrc")
+    subprocess.run(["g++", "-std=c++17", "-shared", "-fPIC", "-I", csrc, "-o", str(d / "plan.so"), str(d / "plan.cpp")],
+                   check=True)
+    so = ctypes.CDLL(str(d / "plan.so"))
+
+    def get(batch, shape, cout, dma):
+        o = (ctypes.c_int * 3)()
+        so.shape(batch, *shape, cout, int(dma), o)
+        return tuple(o)
+    return get
+
+
+# every forward kernel with more tiles than blocks, aligned and not, several
+# slices of input channels, tiles that reach past the lattice and output blocks
+# that pad (80, 112); which kernel a case takes is asserted.  The field, another
+# one in each sample, repeats with a period that no tile divides (in z, where
+# the lattice is a tile deep, it does not repeat), so the checker's output on
+# one period is the whole answer.
+@pytest.mark.parametrize("cin,cout,batch,reps,period,off,kernel", [
+    (32, 32, 4, (3, 3, 2), (11, 21, 25), 0, (2, 8, 16)), (48, 16, 4, (3, 3, 2), (11, 21, 25), 0, (1, 8, 16)),
+    (32, 32, 9, (5, 3, 1), (13, 19, 8), 0, (2, 8, 8)), (48, 16, 9, (5, 3, 1), (13, 19, 8), 0, (1, 8, 8)),
+    (32, 64, 4, (2, 3, 2), (9, 11, 25), 0, (4, 4, 16)), (48, 112, 4, (2, 3, 2), (9, 11, 25), 0, (4, 4, 16)),
+    (32, 48, 4, (2, 3, 2), (9, 11, 25), 0, (3, 4, 16)), (48, 32, 4, (2, 3, 2), (9, 11, 25), 0, (2, 4, 16)),
+    (32, 16, 4, (2, 3, 2), (9, 11, 25), 0, (1, 4, 16)), (32, 64, 12, (3, 2, 1), (13, 19, 8), 0, (4, 4, 8)),
+    (32, 80, 12, (3, 2, 1), (13, 19, 8), 0, (3, 4, 8)), (48, 32, 12, (3, 2, 1), (13, 19, 8), 0, (2, 4, 8)),
+    (32, 16, 12, (3, 2, 1), (13, 19, 8), 0, (1, 4, 8)),
+    (32, 64, 4, (2, 3, 2), (9, 11, 25), 1, (4, 4, 16)), (48, 80, 4, (2, 3, 2), (9, 11, 25), 1, (3, 4, 16)),
+    (48, 32, 4, (3, 3, 2), (11, 21, 25), 1, (2, 4, 16)), (32, 16, 4, (3, 3, 2), (11, 21, 25), 1, (1, 4, 16)),
+    (32, 112, 12, (3, 2, 1), (13, 19, 8), 1, (4, 4, 8)), (32, 48, 12, (3, 2, 1), (13, 19, 8), 1, (3, 4, 8)),
+    (48, 32, 12, (3, 2, 1), (13, 19, 8), 1, (2, 4, 8)), (32, 16, 12, (3, 2, 1), (13, 19, 8), 1, (1, 4, 8))])
+def test_conv_forward_kernels(conv_shape, cin, cout, batch, reps, period, off, kernel):
+    shape = tuple(a * b for a, b in zip(reps, period))
+    assert conv_shape(batch, shape, cout, not off) == kernel
+    lib = L.lib()
+    rng = np.random.default_rng(cin + 3 * cout + batch)
+    m, n = int(np.prod(period)), batch * int(np.prod(shape))
+
+    def whole(a, c):
+        return np.ascontiguousarray(np.tile(a.reshape((batch,) + period + (c,)), (1,) + reps + (1,))).ravel()
+
+    x, w = bf16_round(rng.standard_normal(batch * m * cin)), bf16_round(rng.standard_normal(27 * cout * cin))
+    bias = rng.standard_normal(cout).astype(np.float32)
+    pad = np.zeros(4 * off, np.uint16)
+    dx = dev(np.concatenate([pad, whole(bf16_bits(x), cin)]), np.uint16)
+    dw, db = dev(np.concatenate([pad, bf16_bits(w)]), np.uint16), dev(bias, np.float32)
+    y, z, a, a1 = (L.DeviceArray(n * cout, t) for t in (np.float32, np.float32, np.uint16, np.uint16))
+    print(f"forward kernel {kernel} cin={cin} cout={cout} batch={batch} shape={shape} off={off}", flush=True)
+    at_ = (at(dx, 8 * off), at(dw, 8 * off), vp(db))
+    want = O.conv3_fwd(x, w, bias.astype(np.float64), period, cin, cout, batch)
+    mag = O.conv3_fwd(np.abs(x), np.abs(w), np.abs(bias.astype(np.float64)), period, cin, cout, batch)
+    want, bound = whole(want, cout), whole(2 * (27 * cin + 2) * EPS32 * mag + 1e-30, cout)
+    assert lib.ldw_conv3d_fwd(*at_, vp(y), batch, *shape, cin, cout, 0) == 0
+    got = y.download()
+    within(got.astype(np.float64), want, bound, "forward")
+    assert lib.ldw_conv3d_fwd_silu(*at_, vp(z), vp(a), batch, *shape, cin, cout) == 0
+    assert np.array_equal(z.download(), got)
+    assert lib.ldw_nn_silu_fwd(vp(y), vp(a1), n * cout) == 0
+    assert np.array_equal(a.download(), a1.download())
+    assert lib.ldw_conv3d_fwd(*at_, vp(y), batch, *shape, cin, cout, 1) == 0
+    within(y.download().astype(np.float64), 2 * want, 2 * bound, "accumulated")
 
 
 # operands off 16-byte alignment are read where they are: no copy is kept
