@@ -672,6 +672,7 @@ hipError_t launch_conv3_fwd(const uint16_t * x, const uint16_t * w, const float 
   }
   else {
     switch (c.nt) {
+    case 6: CONV_4(6); break;
     case 4: CONV_4(4); break;
     case 3: CONV_4(3); break;
     case 2: CONV_4(2); break;

@@ -23,6 +23,11 @@ struct ConvShape { int nt, ty, zt; };
 // with 4), and fewer where the grid would not give each CU two blocks (64 ->
 // 64 on 8 x 16^3: 22 us with nt = 4, 17 with 2 or 1).
 //
+// Multiples of 96 channels take 6 blocks of 16 where that makes enough blocks:
+// the halo is staged once instead of twice, and 24 LDS reads serve 72 MFMAs
+// (15 serve 36 with nt = 3).  160 -> 96 on 64^3: 198 us with nt = 6, 229 with 3;
+// 96 -> 96 on 4 x 33x47x65: 256 us.
+//
 // Misaligned operands (dma = 0) take 4 rows, which halves the kernels built
 // for them.
 inline ConvShape conv_shape(int batch, int nx, int ny, int nz, int nb16, bool dma) {
@@ -40,6 +45,7 @@ inline ConvShape conv_shape(int batch, int nx, int ny, int nz, int nb16, bool dm
   else {
     c.nt = ((nb16 + 3)/4*4 <= (nb16 + 2)/3*3) ? 4 : 3;
   }
+  if (nb16 % 6 == 0 && tiles(4)*(nb16/6) >= CONV_BLOCKS) c.nt = 6;
   while (c.nt > 1 && tiles(c.ty)*((nb16 + c.nt - 1)/c.nt) < CONV_BLOCKS) c.nt--;
   return c;
 }

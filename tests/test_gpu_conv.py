@@ -166,6 +166,8 @@ extern "C" void shape(int b, int nx, int ny, int nz, int cout, int dma, int * o)
     (32, 16, 4, (2, 3, 2), (9, 11, 25), 0, (1, 4, 16)), (32, 64, 12, (3, 2, 1), (13, 19, 8), 0, (4, 4, 8)),
     (32, 80, 12, (3, 2, 1), (13, 19, 8), 0, (3, 4, 8)), (48, 32, 12, (3, 2, 1), (13, 19, 8), 0, (2, 4, 8)),
     (32, 16, 12, (3, 2, 1), (13, 19, 8), 0, (1, 4, 8)),
+    (32, 96, 4, (2, 3, 2), (9, 11, 25), 0, (6, 4, 16)), (48, 96, 12, (3, 2, 1), (13, 19, 8), 0, (6, 4, 8)),
+    (32, 96, 4, (2, 3, 2), (9, 11, 25), 1, (6, 4, 16)), (32, 96, 12, (3, 2, 1), (13, 19, 8), 1, (6, 4, 8)),
     (32, 64, 4, (2, 3, 2), (9, 11, 25), 1, (4, 4, 16)), (48, 80, 4, (2, 3, 2), (9, 11, 25), 1, (3, 4, 16)),
     (48, 32, 4, (3, 3, 2), (11, 21, 25), 1, (2, 4, 16)), (32, 16, 4, (3, 3, 2), (11, 21, 25), 1, (1, 4, 16)),
     (32, 112, 12, (3, 2, 1), (13, 19, 8), 1, (4, 4, 8)), (32, 48, 12, (3, 2, 1), (13, 19, 8), 1, (3, 4, 8)),
