@@ -71,10 +71,10 @@ typedef uint16_t h4a __attribute__((ext_vector_type(4), aligned(2)));
 // lane (r, q) ends with channels 4q .. 4q+3 of position r: 16-byte stores.
 //
 // Bound by the halo loads beside the MFMAs (which are busy 42 % of the time):
-// without them 80 -> 32 channels on 8 x 64^3 would take 264 us.  It takes 357 us
-// (813 TFLOP/s) and the network's 12 layers on 8 x 64^3 0.95 ms, against 500 us
-// and 1.63 ms for a tile per block, staged through registers with two
-// barriers per three taps and a read per tap.
+// without them 80 -> 32 channels on 8 x 64^3 would take 264 us.  It takes 342 us
+// (847 TFLOP/s), 373 with the SiLU, and the network's 12 layers on 8 x 64^3 1.01
+// ms, against 500 us and 1.62 ms for a tile per block, staged through registers
+// with two barriers per three taps and a read per tap.
 
 constexpr int NUNIT = 5;
 constexpr int NXCD = 8;
